@@ -38,6 +38,7 @@ CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", f"-I
 HIP_SOURCES = [
     CSRC / "hipabi" / "gdb_hip.cpp",
     CSRC / "hipabi" / "gdb_kernels.cpp",
+    CSRC / "hipabi" / "gdb_group_rows.cpp",
 ]
 ENGINE_DIRS = ["core", "operators", "planning", "execution", "infra", "runtime"]
 

@@ -631,8 +631,10 @@ gdb_status gdb_result_column_format(gdb_result r, int idx, int* scale, int* is_d
 gdb_status gdb_result_i64(gdb_result r, int idx, int64_t* out) {
     const auto& c = r->r.columns.at(static_cast<size_t>(idx));
     if (c.type != ResultColumn::I64) return setErr(GDB_ERR_INVALID, "gdb_result_i64: column is not int64");
-    std::memcpy(out, c.i64.data(), c.i64.size() * 8);
-    return GDB_OK;
+    return guard([&]() -> gdb_status {
+        c.copyI64(out);
+        return GDB_OK;
+    });
 }
 
 gdb_status gdb_result_i128(gdb_result r, int idx, int64_t* out) {

@@ -587,7 +587,117 @@ std::vector<std::array<uint64_t, 4>> HipGenericExecutor::checkStatus(const HipCo
     return judgeStatuses(ps);
 }
 
-GenericResult HipGenericExecutor::collectResult(const HipCodegen& cg) const {
+void HipGenericExecutor::freeWorkspace(Workspace& w) {
+    if (w.ptr) gdb_free(ctx_, w.ptr);  // waits for what still uses it
+    w = Workspace{};
+}
+
+bool HipGenericExecutor::ensureWorkspace(Workspace& w, size_t bytes) {
+    if (bytes <= w.bytes) return true;
+    freeWorkspace(w);
+    if (gdb_alloc(ctx_, bytes, &w.ptr) != GDB_OK) {
+        w = Workspace{};
+        return false;
+    }
+    w.bytes = bytes;
+    return true;
+}
+
+std::shared_ptr<void> HipGenericExecutor::stagingFor(size_t bytes) {
+    if (staging_ && staging_.use_count() == 1 && stagingBytes_ >= bytes) return staging_;
+    if (bytes <= kKeepStaging) staging_.reset();
+    void* h = nullptr;
+    if (gdb_host_alloc_pinned(bytes, &h) != GDB_OK) return nullptr;
+    std::shared_ptr<void> p(h, [](void* q) { gdb_host_free_pinned(q); });
+    if (bytes <= kKeepStaging) {
+        staging_ = p;
+        stagingBytes_ = bytes;
+    }
+    return p;
+}
+
+// The groups of a hash-aggregate table, ordered and split into columns on the
+// device, so only the result crosses the link (32 bytes a group instead of 32
+// a slot, from pinned memory) and the host sorts nothing. A group-by of 40M
+// rows with 2.2M groups in 8M slots took 392 ms with the table copied and
+// sorted on the host, 4.9 ms so; 8M rows with 400K groups 82 and 1.4 ms.
+// Tables of at most 2 * GDB_GROUP_ROWS_SMALL slots take one launch of one
+// block that writes the rows to pinned memory itself; a larger one would keep
+// that block busy longer than the general path's dozen launches take. False
+// when the workspace cannot be had (the caller reads the table instead).
+bool HipGenericExecutor::collectGroups(const HipResultSchema& schema, GenericResult& res) {
+    const auto& h = schema.hash;
+    const auto it = buffers_.find(h.tableName);
+    if (h.slotWords != 4 || it == buffers_.end()) return false;
+    const uint64_t slots = sizes_.resolve(h.slotsSymbol);
+    if (slots > kMaxGroupSlots || slots * 32 > it->second.bytes) return false;
+    const uint64_t* table = static_cast<const uint64_t*>(it->second.ptr);
+    static const char* const names[4] = {"count", "sum", "min", "max"};
+    res.columns.assign(5, ResultColumn{});
+    res.columns[0].name = h.keyName;
+    for (size_t k = 0; k < 4; ++k) res.columns[k + 1].name = names[k];
+
+    if (slots <= 2 * GDB_GROUP_ROWS_SMALL) {
+        auto out = stagingFor(GDB_GROUP_ROWS_SMALL_BYTES);
+        if (!out) return false;
+        uint64_t* w = static_cast<uint64_t*>(out.get());
+        check(gdb_group_rows_small(table, slots, w, stream_), "gdb_group_rows_small");
+        check(gdb_stream_sync(stream_), "gdb_stream_sync");
+        const size_t n = static_cast<size_t>(w[0]);
+        if (n <= GDB_GROUP_ROWS_SMALL) {
+            const uint64_t* col = w + 8;
+            for (auto& c : res.columns) c.i64.resize(n);
+            for (size_t r = 0; r < n; ++r) {
+                res.columns[0].i64[r] = static_cast<int64_t>(col[r] & 0xFFFFFFFFull);
+                res.columns[1].i64[r] = static_cast<int64_t>(col[r] >> 32);
+            }
+            for (size_t k = 1; k < 4; ++k)
+                std::memcpy(res.columns[k + 1].i64.data(), col + k * GDB_GROUP_ROWS_SMALL, n * 8);
+            return true;
+        }
+    }
+
+    // workspaces: head | pairs; once the number of groups is known, sort scratch | columns
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    if (!ensureWorkspace(groupPairs_, 256 + static_cast<size_t>(slots) * 8)) return false;
+    uint64_t* const head = static_cast<uint64_t*>(groupPairs_.ptr);
+    uint64_t* const pairs = head + 32;
+    uint64_t* host = ensurePinned(16);
+    check(gdb_group_rows_compact(table, slots, pairs, head, stream_), "gdb_group_rows_compact");
+    check(gdb_memcpy_d2h_async(host, head, 16, stream_), "read group count");
+    check(gdb_stream_sync(stream_), "gdb_stream_sync");
+    const uint64_t n = host[0], maxKey = host[1];
+    if (n == 0) return true;
+    const size_t col8 = up(static_cast<size_t>(n) * 8), col4 = up(static_cast<size_t>(n) * 4);
+    const size_t scratch = up(gdb_group_rows_scratch_bytes(n)), colBytes = 3 * col8 + 2 * col4;
+    if (!ensureWorkspace(groupCols_, scratch + colBytes)) return false;
+    auto out = stagingFor(colBytes);
+    if (!out) return false;
+    char* const cols = static_cast<char*>(groupCols_.ptr) + scratch;
+    const size_t at[5] = {3 * col8, 3 * col8 + col4, 0, col8, 2 * col8};  // key, count, sum, min, max
+    check(gdb_group_rows_sort(table, pairs, n, maxKey, groupCols_.ptr, reinterpret_cast<uint32_t*>(cols + at[0]),
+                              reinterpret_cast<uint32_t*>(cols + at[1]), reinterpret_cast<int64_t*>(cols + at[2]),
+                              reinterpret_cast<int64_t*>(cols + at[3]), reinterpret_cast<int64_t*>(cols + at[4]), stream_),
+          "gdb_group_rows_sort");
+    check(gdb_memcpy_d2h_async(out.get(), cols, colBytes, stream_), "read group columns");
+    check(gdb_stream_sync(stream_), "gdb_stream_sync");
+    for (size_t k = 0; k < 5; ++k) {
+        auto& c = res.columns[k];
+        c.hold = out;
+        c.raw = static_cast<const char*>(out.get()) + at[k];
+        c.raw32 = k < 2;
+        c.rawRows = static_cast<size_t>(n);
+    }
+    if (groupPairs_.bytes > kKeepWorkspace) freeWorkspace(groupPairs_);
+    if (groupCols_.bytes > kKeepWorkspace) freeWorkspace(groupCols_);
+    return true;
+}
+
+GenericResult HipGenericExecutor::collectResult(const HipCodegen& cg) {
+    if (cg.getResultSchema().kind == HipResultSchema::HASH_AGG) {
+        GenericResult res;
+        if (collectGroups(cg.getResultSchema(), res)) return res;
+    }
     check(gdb_stream_sync(stream_), "gdb_stream_sync");
     return HipResultCollector::collect(
         cg.getResultSchema(),
@@ -599,6 +709,10 @@ void HipGenericExecutor::releaseAllocatedBuffers() {
     for (auto& kv : buffers_)
         if (kv.second.owned && kv.second.ptr) gdb_free(ctx_, kv.second.ptr);
     buffers_.clear();
+    freeWorkspace(groupPairs_);
+    freeWorkspace(groupCols_);
+    staging_.reset();
+    stagingBytes_ = 0;
 }
 
 void* HipGenericExecutor::getAllocatedBuffer(const std::string& name) const {
@@ -612,7 +726,7 @@ size_t HipGenericExecutor::getAllocatedBytes(const std::string& name) const {
 }
 
 size_t HipGenericExecutor::ownedBytes() const {
-    size_t n = 0;
+    size_t n = groupPairs_.bytes + groupCols_.bytes;
     for (const auto& kv : buffers_)
         if (kv.second.owned) n += kv.second.bytes;
     return n;

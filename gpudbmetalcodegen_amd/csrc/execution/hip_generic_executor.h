@@ -22,6 +22,7 @@
 #include <array>
 #include <functional>
 #include <map>
+#include <memory>
 #include <stdexcept>
 #include <string>
 #include <unordered_map>
@@ -143,7 +144,7 @@ public:
     PendingStatus enqueueStatus(const HipCodegen& cg, int firstPhase = 0, int lastPhase = -1);
     std::vector<std::array<uint64_t, 4>> judgeStatuses(const PendingStatus& ps) const;
 
-    GenericResult collectResult(const HipCodegen& cg) const;
+    GenericResult collectResult(const HipCodegen& cg);
     void releaseAllocatedBuffers();
     void* getAllocatedBuffer(const std::string& name) const;
     size_t getAllocatedBytes(const std::string& name) const;
@@ -193,6 +194,24 @@ private:
     std::vector<const void*> statusPtrCache_;
     uint64_t* ensurePinned(size_t bytes);
     std::map<std::pair<gdb_kernel, int>, int> occupancy_;
+    // Hash-aggregate results (collectGroups): device workspaces, grown as
+    // needed and freed with the runner's buffers, and the pinned block the
+    // last result was read into, shared with that result and reused when it
+    // is gone. Anything larger than these goes when its result is made.
+    static constexpr size_t kKeepWorkspace = size_t{1} << 30;
+    static constexpr size_t kKeepStaging = size_t{256} << 20;
+    static constexpr uint64_t kMaxGroupSlots = uint64_t{1} << 31;
+    struct Workspace {
+        void* ptr = nullptr;
+        size_t bytes = 0;
+    };
+    Workspace groupPairs_, groupCols_;
+    std::shared_ptr<void> staging_;
+    size_t stagingBytes_ = 0;
+    bool ensureWorkspace(Workspace& w, size_t bytes);
+    void freeWorkspace(Workspace& w);
+    std::shared_ptr<void> stagingFor(size_t bytes);
+    bool collectGroups(const HipResultSchema& schema, GenericResult& res);
     bool skipInit_ = false;
     bool phaseTiming_ = true;
     std::vector<std::string> lateSymbols_;

@@ -2,9 +2,11 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cstring>
 #include <numeric>
 #include <sstream>
 #include <stdexcept>
+#include <thread>
 
 namespace gdb {
 namespace codegen {
@@ -55,6 +57,30 @@ std::string csvField(const std::string& s) {
 
 }  // namespace
 
+void ResultColumn::copyI64(int64_t* out) const {
+    if (!raw) {
+        if (!i64.empty()) std::memcpy(out, i64.data(), i64.size() * 8);
+        return;
+    }
+    auto part = [&](size_t b, size_t e) {
+        if (!raw32) {
+            std::memcpy(out + b, static_cast<const int64_t*>(raw) + b, (e - b) * 8);
+            return;
+        }
+        const uint32_t* v = static_cast<const uint32_t*>(raw);
+        for (size_t r = b; r < e; ++r) out[r] = static_cast<int64_t>(v[r]);
+    };
+    // a thread costs ~20 us to start, 256K values ~0.5-1 ms to write to fresh pages
+    const size_t threads = std::min<size_t>(8, rawRows / (1u << 18));
+    if (threads < 2) return part(0, rawRows);
+    std::vector<std::thread> pool;
+    const size_t step = (rawRows + threads - 1) / threads;
+    for (size_t t = 1; t < threads; ++t)
+        pool.emplace_back(part, std::min(rawRows, t * step), std::min(rawRows, (t + 1) * step));
+    part(0, step);
+    for (auto& th : pool) th.join();
+}
+
 const ResultColumn& GenericResult::column(const std::string& name) const {
     for (const auto& c : columns)
         if (c.name == name) return c;
@@ -73,9 +99,9 @@ std::string GenericResult::toCanonical() const {
             if (col.type == ResultColumn::STR)
                 os << csvField(col.str[r]);
             else if (col.date)
-                os << dateString(col.type == ResultColumn::I64 ? col.i64[r] : static_cast<int64_t>(col.i128[r]));
+                os << dateString(col.type == ResultColumn::I64 ? col.i64At(r) : static_cast<int64_t>(col.i128[r]));
             else
-                os << fixedToString(col.type == ResultColumn::I64 ? col.i64[r] : col.i128[r], col.scale);
+                os << fixedToString(col.type == ResultColumn::I64 ? col.i64At(r) : col.i128[r], col.scale);
         }
         os << "\n";
     }

@@ -11,6 +11,7 @@
 
 #include <cstdint>
 #include <functional>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -26,7 +27,23 @@ struct ResultColumn {
     std::vector<std::string> str;
     int scale = 0;      // integer columns: fixed-point digits, shown as an exact decimal
     bool date = false;  // integer columns: YYYYMMDD shown as YYYY-MM-DD
-    size_t size() const { return type == I64 ? i64.size() : (type == I128 ? i128.size() : str.size()); }
+    // A column of many groups as it came from the device (I64 only; i64 is
+    // empty then): rawRows values of 64 bits, or 32 bits unsigned, in memory
+    // that `hold` keeps. Widened once, into the caller's array.
+    std::shared_ptr<const void> hold;
+    const void* raw = nullptr;
+    bool raw32 = false;
+    size_t rawRows = 0;
+    size_t size() const {
+        return type == I64 ? (raw ? rawRows : i64.size()) : (type == I128 ? i128.size() : str.size());
+    }
+    int64_t i64At(size_t r) const {
+        if (!raw) return i64[r];
+        return raw32 ? static_cast<int64_t>(static_cast<const uint32_t*>(raw)[r]) : static_cast<const int64_t*>(raw)[r];
+    }
+    // All values of an I64 column; large ones are copied by several threads
+    // (fresh pages of the caller's array cost more than the copy itself).
+    void copyI64(int64_t* out) const;
 };
 
 struct GenericResult {

@@ -63,6 +63,30 @@ gdb_status gdb_gen_device_uniform_i64(int64_t* out, uint64_t n, int64_t lo, int6
  * the reference (its runner reads status per query from shared memory). */
 gdb_status gdb_gather_words(const uint64_t* const* src, int n, int words, uint64_t* dst, gdb_stream st);
 
+/* Groups of a hash-aggregate table in key order, as columns: slots of 4 words
+ * [key | count << 32, sum, min, max], empty key 0xFFFFFFFF (the result the
+ * reference's collector assembles on the host,
+ * codegen/execution/metal_result_collector.cpp:228-235).
+ *
+ * Small tables (at most 2 * GDB_GROUP_ROWS_SMALL slots) in one launch: word 0
+ * of pinned_out receives the number of groups n; when n <=
+ * GDB_GROUP_ROWS_SMALL, the groups' four slot words follow from word 8 as four
+ * arrays of GDB_GROUP_ROWS_SMALL words. pinned_out is pinned host memory of
+ * GDB_GROUP_ROWS_SMALL_BYTES, read after the stream is waited for.
+ *
+ * Others in two steps: compact writes the occupied slots to pairs (room for
+ * `slots` words), their number to head[0] and the largest key to head[1]
+ * (device memory); with both known on the host, sort orders the pairs (using
+ * gdb_group_rows_scratch_bytes(n) of scratch) and writes n-element columns. */
+#define GDB_GROUP_ROWS_SMALL 8192
+#define GDB_GROUP_ROWS_SMALL_BYTES ((8 + 4 * GDB_GROUP_ROWS_SMALL) * 8)
+const char* gdb_group_rows_last_error(void);
+gdb_status gdb_group_rows_small(const uint64_t* table, uint64_t slots, uint64_t* pinned_out, gdb_stream s);
+gdb_status gdb_group_rows_compact(const uint64_t* table, uint64_t slots, uint64_t* pairs, uint64_t* head, gdb_stream s);
+size_t gdb_group_rows_scratch_bytes(uint64_t n);
+gdb_status gdb_group_rows_sort(const uint64_t* table, uint64_t* pairs, uint64_t n, uint64_t max_key, void* scratch,
+                               uint32_t* key, uint32_t* count, int64_t* sum, int64_t* mn, int64_t* mx, gdb_stream s);
+
 /* Streaming device copy (16-byte aligned pointers and size). */
 gdb_status gdb_copy_async(void* dst, const void* src, size_t bytes, gdb_stream st);
 

@@ -1,0 +1,65 @@
+"""A hash-aggregate table's groups ordered and split into columns on the
+device (the result of every group-by): against the oracle at the sizes where
+the one-block form, the sort's tiles and its digit passes end."""
+
+import numpy as np
+import pytest
+
+import oracle
+from gpudbmetalcodegen_amd import queries as Q
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ctx, keys, slots, variant="global"):
+    r = np.random.default_rng(len(keys))
+    keys = r.permutation(np.concatenate([keys, keys[: len(keys) // 3]])).astype(np.int64)
+    G = {"g_key": keys.astype(np.uint32).view(np.int32), "g_val": r.integers(-10**12, 10**12, keys.size)}
+    dev = Q.upload_tables(ctx, {"G": G})
+    try:
+        run = Q.run_groupby(ctx, dev, slots=slots, variant=variant, lds_slots=1024)
+        exp = oracle.groupby(G)
+        order = np.argsort(np.asarray(exp["key"]).astype(np.int64) & 0xFFFFFFFF)
+        for c in ("key", "count", "sum", "min", "max"):
+            e = np.asarray(exp[c])[order]
+            if c == "key":
+                e = e.astype(np.int64) & 0xFFFFFFFF
+            assert run.result.columns[c].dtype == np.int64
+            assert np.array_equal(run.result.columns[c], e), c
+        again = run.executor.collect(run.plan)     # the workspaces and the pinned block are used again
+        assert all(np.array_equal(again.columns[c], run.result.columns[c]) for c in again.columns)
+    finally:
+        dev["G"].free(ctx)
+
+
+# groups around the one-block form's 8,192 rows (16,384 slots) and the sort's 4,096-pair tiles
+@pytest.mark.parametrize("groups,slots", [(1, 64), (63, 128), (700, 2048), (4096, 8192), (8192, 16384), (8193, 16384),
+                                          (12_000, 16384), (100, 32768), (4095, 65536), (4097, 65536), (70_001, 1 << 18)])
+def test_groups_in_key_order(ctx, groups, slots):
+    print(groups, slots, flush=True)
+    _check(ctx, np.arange(1, groups + 1) * 3 + 7, slots)
+
+
+# largest keys that need one to four 8-bit passes, and the ends of the key range
+@pytest.mark.parametrize("top", [200, 40_000, 9_000_000, 2**31 - 1, 2**32 - 2])
+def test_key_ranges(ctx, top):
+    print(top, flush=True)
+    r = np.random.default_rng(top)
+    keys = np.unique(np.concatenate([[0, top], r.integers(0, top, 20_000)]))
+    _check(ctx, keys, 1 << 16)
+
+
+def test_large_result_is_held_apart_from_the_next(ctx):
+    n = 600_000
+    G = {"g_key": np.random.default_rng(3).permutation(n).astype(np.int32), "g_val": np.arange(n, dtype=np.int64)}
+    dev = Q.upload_tables(ctx, {"G": G})
+    try:
+        a = Q.run_groupby(ctx, dev, slots=2 * n, variant="part", lds_slots=1024)
+        first = {k: v.copy() for k, v in a.result.columns.items()}
+        b = Q.run_groupby(ctx, dev, slots=2 * n, variant="part", lds_slots=1024, val_cut=1000, executor=a.executor)
+        assert all(np.array_equal(a.result.columns[c], first[c]) for c in first)
+        assert np.array_equal(first["key"], np.arange(n)) and np.array_equal(np.sort(first["sum"]), np.arange(n))
+        assert b.result.rows() == 1000
+        a.executor.release()
+    finally:
+        dev["G"].free(ctx)
