@@ -1786,25 +1786,33 @@ void HipHashGroupBy::produceImpl(HipCodegen& cg, ConsumerFn consume) {
         if (partialsMax_.empty()) {
             emitLdsGbFlush(cg, T, tab, LS);
         } else {
-            const std::string PT = T + "_pt", PN = T + "_ptn", NP = "nparts_" + T;
-            cg.addBufferParam(PT, "u64", 8, "(" + partialsMax_ + ") * " + CAP + " * 4", InitKind::None, {}, false, true);
-            cg.addBufferParam(PN, "u64", 8, "1", InitKind::Zero, {}, false, true);
+            const std::string PT = T + "_pt", PM = T + "_ptm", PN = T + "_ptn", NP = "nparts_" + T;
+            cg.addBufferParam(PT, "u64", 8, "(" + partialsMax_ + ") * " + s(4LL * ldsSlots_), InitKind::None, {}, false, true);
+            cg.addBufferParam(PM, "u64", 8, "(" + partialsMax_ + ") * " + s(ldsSlots_ / 64), InitKind::None, {}, false, true);
+            cg.addBufferParam(PN, "u64", 8, "2", InitKind::Zero, {}, false, true);
             cg.addSymbolParam(NP, partialsMax_);
-            cg.addComment("the LDS table becomes partial table _pi (word-major, " + CAP + " slots apart), if one is left");
+            cg.addComment("the LDS table becomes partial table _pi, if one is left");
             cg.declareLds("u64", "_pti_" + T, "1");
-            cg.addLine("if (threadIdx.x == 0) _pti_" + T + "[0] = __hip_atomic_fetch_add(" + PN +
-                       ", 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);");
+            // a launch of a few blocks merges each key a few times: the fold
+            // would cost more than it saves (measured in the plan builder)
+            const std::string take = "__hip_atomic_fetch_add(" + PN + ", 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)";
+            cg.addLine("if (threadIdx.x == 0) _pti_" + T + "[0] = " +
+                       (cg.rangeMode() ? take : "gridDim.x < " + s(kMinFoldBlocks) + "u ? ~0ull : " + take) + ";");
             cg.addLine("__syncthreads();");
             cg.addLine("const u64 _pi_" + T + " = _pti_" + T + "[0];");
             cg.addBlock("if (_pi_" + T + " < " + NP + ")", [&]() {
-                cg.addComment("key words of every slot; the other words of occupied slots only");
-                cg.addLine("u64* const _pd = " + PT + " + _pi_" + T + " * " + CAP + "ull * 4ull;");
+                cg.addComment("occupied slots only, 32 bytes each in place, and a bit per slot that says which");
+                cg.addLine("u64x2* const _pd = reinterpret_cast<u64x2*>(" + PT + " + _pi_" + T + " * " +
+                           s(4LL * ldsSlots_) + "ull);");
+                cg.addLine("u64* const _pm = " + PM + " + _pi_" + T + " * " + s(ldsSlots_ / 64) + "ull;");
                 cg.addBlock("for (int _s = (int)threadIdx.x; _s < " + LS + "; _s += (int)blockDim.x)", [&]() {
                     cg.addLine("const u64 _w0 = " + tab + "[_s];");
-                    cg.addLine("_pd[_s] = _w0;");
-                    cg.addBlock("if ((u32)_w0 != GDB_EMPTY_KEY)", [&]() {
-                        cg.addLine("_pd[" + LS + " + _s] = " + tab + "[" + LS + " + _s]; _pd[2 * " + LS + " + _s] = " + tab +
-                                   "[2 * " + LS + " + _s]; _pd[3 * " + LS + " + _s] = " + tab + "[3 * " + LS + " + _s];");
+                    cg.addLine("const bool _oc = (u32)_w0 != GDB_EMPTY_KEY;");
+                    cg.addLine("const u64 _mk = __ballot(_oc);");
+                    cg.addLine("if (gdb_lane() == 0) _pm[_s >> 6] = _mk;");
+                    cg.addBlock("if (_oc)", [&]() {
+                        cg.addLine("_pd[2 * _s] = u64x2{_w0, " + tab + "[" + LS + " + _s]};");
+                        cg.addLine("_pd[2 * _s + 1] = u64x2{" + tab + "[2 * " + LS + " + _s], " + tab + "[3 * " + LS + " + _s]};");
                     });
                 });
             });
@@ -1830,54 +1838,90 @@ void HipGroupByMerge::produceImpl(HipCodegen& cg, ConsumerFn consume) {
     if (ldsSlots_ < 64 || (ldsSlots_ & (ldsSlots_ - 1)))
         throw std::runtime_error("HipGroupByMerge: LDS slots must be a power of two >= 64");
     const std::string st = bindGroupTable(cg, T, slots_);
-    const std::string PT = T + "_pt", PN = T + "_ptn", NP = "nparts_" + T;
-    cg.addBufferParam(PT, "u64", 8, "(" + partialsMax_ + ") * " + CAP + " * 4", InitKind::None, {}, true, true);
-    cg.addBufferParam(PN, "u64", 8, "1", InitKind::Zero, {}, true, true);
+    const std::string PT = T + "_pt", PM = T + "_ptm", PN = T + "_ptn", NP = "nparts_" + T;
+    cg.addBufferParam(PT, "u64", 8, "(" + partialsMax_ + ") * " + s(4LL * ldsSlots_), InitKind::None, {}, true, true);
+    cg.addBufferParam(PM, "u64", 8, "(" + partialsMax_ + ") * " + s(ldsSlots_ / 64), InitKind::None, {}, true, true);
+    cg.addBufferParam(PN, "u64", 8, "2", InitKind::Zero, {}, false, true);
     cg.addSymbolParam(NP, partialsMax_);
     cg.setPhaseRowsExpr("(" + partialsMax_ + ") * " + CAP);
-    cg.addComment("GroupByMerge " + T + ": partial LDS tables -> one LDS table per block -> the global table");
+    cg.addComment("GroupByMerge " + T + ": a block takes a range of home slots over every partial table, so each key "
+                  "reaches the global table once");
     cg.declareLds("u64", tab, CAP + " * 4");
     std::string LS, LB;
     std::tie(LS, LB) = ldsTableSize(cg, T, ldsSlots_, ldsBitsScalar_);
-    emitLdsGbInit(cg, tab, LS);
-    cg.addLine("__syncthreads();");
     cg.addLine("const u64 _np = " + PN + "[0] < " + NP + " ? " + PN + "[0] : " + NP + ";");
-    cg.addLine("const u64 _flat = _np * " + CAP + "ull;  // partial slots written");
-    auto body = [&]() {
-        cg.addLine("const u64 _s = _r & " + s(ldsSlots_ - 1) + "ull;");
-        cg.addBlock("if (_s < (u64)" + LS + ")", [&]() {
-            cg.addLine("const u64* const _p = " + PT + " + (_r - _s) * 4ull + _s;");
-            cg.addLine("const u64 _w0 = _p[0];");
-            cg.addBlock("if ((u32)_w0 != GDB_EMPTY_KEY)", [&]() {
-                cg.addLine("const u32 _k = (u32)_w0, _c = (u32)(_w0 >> 32);");
-                cg.addLine("const i64 _sm = (i64)_p[" + LS + "], _mn = (i64)_p[2 * " + LS + "], _mx = (i64)_p[3 * " + LS +
-                           "];");
-                // a bounded probe window: with more groups than LDS slots a
-                // full-table probe per missing key would cost thousands of
-                // LDS loads; such keys merge into the global table instead
-                cg.addBlock("if (gdb_lds_gb_merge_at(" + tab + ", (u32)" + LS + " - 1u, (u32)gdb_hash_slot(_k, " + LB +
-                                "), _k, _c, _sm, _mn, _mx, " + s(kMergeWindow) + "u) < 0)",
-                            [&]() {
-                                cg.addLine("const int _g = gdb_gb_merge(" + T + ", _bits_" + T +
-                                           ", _k, _c, _sm, _mn, _mx, _maxp_" + T + ");");
-                                cg.addLine("if (_g < 0) ++_ovf_" + T + "; else _ins_" + T + " += (u32)_g;");
-                            });
+    cg.addBlock("if (_np != 0)", [&]() {
+        if (cg.rangeMode()) {
+            cg.addComment("work item: units [_rb, _re) of nparts x slots, i.e. the home slots they scale to");
+            cg.addLine("const u64 _un = " + NP + " * " + CAP + "ull;");
+            cg.addLine("const u32 _h0 = (u32)(_rb * (u64)" + LS + " / _un), _h1 = (u32)((_re < _un ? _re : _un) * (u64)" + LS +
+                       " / _un);");
+        } else {
+            cg.addLine("const u32 _h0 = (u32)((u64)blockIdx.x * (u64)" + LS + " / gridDim.x), _h1 = (u32)(((u64)blockIdx.x + 1) * (u64)" +
+                       LS + " / gridDim.x);");
+        }
+        cg.addLine("const u32 _len = _h1 - _h0, _lm = (u32)" + LS + " - 1u;");
+        cg.addComment("LDS table: 4 slots per home slot of the range, indexed by the hash bits below the home slot's");
+        cg.addLine("u32 _mb = 6;");
+        cg.addLine("while (_mb < " + LB + " && (1u << _mb) < 4u * _len) ++_mb;");
+        cg.addLine("const int _ms = 1 << _mb;");
+        emitLdsGbInit(cg, tab, "_ms");
+        cg.addLine("__syncthreads();");
+        cg.addComment("a key sits at most a probe window past its home slot");
+        cg.addLine("const u32 _sc = _len == 0 ? 0u : (_len + " + s(window_ - 1) + "u < (u32)" + LS + " ? _len + " +
+                   s(window_ - 1) + "u : (u32)" + LS + ");");
+        cg.addComment("a lane takes 16 slots of one partial: their occupancy bits, then the occupied slots, four in "
+                      "flight. Lanes stay full whatever the tables hold (a wave over 64 slots of a partial left most of "
+                      "its lanes idle in every LDS merge); neighbouring partials start at different slots, so they "
+                      "seldom meet at one key");
+        cg.addLine("const u32 _qa = " + LS + " < 16 ? 1u : (u32)" + LS + " / 16u;");
+        cg.addLine("const u32 _qn = _sc == 0 ? 0u : ((_h0 & 15u) + _sc + 15u) >> 4, _nq = _qn < _qa ? _qn : _qa;");
+        cg.addLine("const u32 _tot = (u32)_np * _nq;");
+        cg.addBlock("for (u32 _x = threadIdx.x; _x < _tot; _x += blockDim.x)", [&]() {
+            cg.addLine("const u32 _pp = _x / _nq, _qq = ((_h0 >> 4) + (_x - _pp * _nq)) & (_qa - 1u), _rt = _pp & 15u;");
+            cg.addLine("u32 _bits = reinterpret_cast<const u16*>(" + PM + ")[_pp * " + s(ldsSlots_ / 16) + "u + _qq];");
+            cg.addLine("_bits = ((_bits >> _rt) | (_bits << (16u - _rt))) & 0xFFFFu;");
+            cg.addLine("const u64x2* const _e0 = reinterpret_cast<const u64x2*>(" + PT + " + (u64)_pp * " +
+                       s(4LL * ldsSlots_) + "ull) + _qq * 32u;");
+            cg.addBlock("while (_bits != 0)", [&]() {
+                cg.addLine("u64x2 _a[4], _b[4];");
+                cg.addLine("bool _in[4];");
+                cg.addLine("#pragma unroll");
+                cg.addBlock("for (u32 _q = 0; _q < 4; ++_q)", [&]() {
+                    cg.addLine("_in[_q] = _bits != 0;");
+                    cg.addLine("const u32 _j = ((u32)__builtin_ctz(_bits | 0x10000u) + _rt) & 15u;");
+                    cg.addLine("_bits &= _bits - 1u;");
+                    cg.addLine("_a[_q] = _e0[2 * _j]; _b[_q] = _e0[2 * _j + 1];");
+                });
+                cg.addLine("#pragma unroll");
+                cg.addBlock("for (u32 _q = 0; _q < 4; ++_q)", [&]() {
+                    cg.addBlock("if (_in[_q] && (((u32)gdb_hash_slot((u32)_a[_q].x, " + LB + ") - _h0) & _lm) < _len)", [&]() {
+                        cg.addLine("const u32 _k = (u32)_a[_q].x, _c = (u32)(_a[_q].x >> 32);");
+                        cg.addLine("const i64 _sm = (i64)_a[_q].y, _mn = (i64)_b[_q].x, _mx = (i64)_b[_q].y;");
+                        // a bounded probe window: a range with more keys than
+                        // LDS slots merges the rest into the global table
+                        cg.addBlock("if (gdb_lds_gb_merge_at(" + tab + ", (u32)_ms - 1u, ((_k * GDB_KNUTH) << " + LB +
+                                        ") >> (32u - _mb), _k, _c, _sm, _mn, _mx, " + s(kMergeWindow) + "u) < 0)",
+                                    [&]() {
+                                        cg.addLine("const int _g = gdb_gb_merge(" + T + ", _bits_" + T +
+                                                   ", _k, _c, _sm, _mn, _mx, _maxp_" + T + ");");
+                                        cg.addLine("if (_g < 0) ++_ovf_" + T + "; else _ins_" + T + " += (u32)_g;");
+                                    });
+                    });
+                });
             });
         });
-    };
-    if (cg.rangeMode()) {
-        cg.addComment("work item: partial slots [_rb, _re)");
-        cg.addBlock("for (u64 _r = _rb + threadIdx.x; _r < (_re < _flat ? _re : _flat); _r += blockDim.x)", body);
-    } else {
-        cg.addComment("block: contiguous tiles of partial slots, tile-strided over the grid");
-        cg.addLine("const u64 _tile = (u64)blockDim.x * ITEMS;");
-        cg.addBlock("for (u64 _t0 = (u64)blockIdx.x * _tile; _t0 < _flat; _t0 += (u64)gridDim.x * _tile)", [&]() {
-            cg.addLine("const u64 _te = _t0 + _tile < _flat ? _t0 + _tile : _flat;");
-            cg.addBlock("for (u64 _r = _t0 + threadIdx.x; _r < _te; _r += blockDim.x)", body);
-        });
-    }
-    cg.addLine("__syncthreads();");
-    emitLdsGbFlush(cg, T, tab, LS);
+        cg.addLine("__syncthreads();");
+        emitLdsGbFlush(cg, T, tab, "_ms");
+        if (!cg.rangeMode()) {
+            cg.addComment("the partials are folded: the last block forgets them, so a run that adds to the table (no "
+                          "initialisation, chunks) does not fold them again");
+            cg.addLine("__syncthreads();");
+            cg.addBlock("if (threadIdx.x == 0 && __hip_atomic_fetch_add(" + PN +
+                            " + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (u64)gridDim.x - 1ull)",
+                        [&]() { cg.addLine(PN + "[0] = 0; " + PN + "[1] = 0;"); });
+        }
+    });
     cg.addComment("group-by status: [0] overflow flag, [2] keys inserted");
     emitBlockStatus(cg, st, {{"_ins_" + T, 2, false}, {"_ovf_" + T, 0, true}});
     consume();

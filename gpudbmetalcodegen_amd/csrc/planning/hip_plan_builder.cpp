@@ -366,11 +366,30 @@ HipQueryPlan buildGroupBy(const PlanOptions& o) {
                                                variant == "global" ? HipHashGroupBy::GLOBAL : HipHashGroupBy::LDS,
                                                ldsSlots);
     gb->setWindow(optInt(o, "window", 16));
-    auto& ph = appendPhase(plan, "GB_agg", std::move(gb), optInt(o, "block", 512), optInt(o, "items", 4), {4});
-    ph.launchBound = 1024;
+    // LDS variant: the blocks' LDS tables are folded by GB_merge instead of
+    // merged into the group table one by one, which cost the same keys' four
+    // atomics once per block, all on the same lines: 1M rows of 700 groups
+    // took 353 us so, 16 us and a fold of 20 us now. As many partial tables as blocks can
+    // run at once (one per 32 B x lds_slots of a CU's 160 KB, 256 CUs), whatever
+    // the rows, so a chunked run keeps what earlier chunks left. Below 16
+    // blocks there is little to fold and they merge directly.
+    const bool fold = variant == "lds";
+    const int perCu = std::max(1, std::min(4, 155 * 1024 / (32 * ldsSlots)));
+    const std::string pmax = std::to_string(256 * perCu);
+    if (fold) gb->setPartials(pmax);
+    // block 1024: as many waves per CU as two blocks of 512, half the partials
+    // (100M rows 454 us against 556 at 512; 1M 18 us and a fold of 21, against 20 and 32)
+    appendPhase(plan, "GB_agg", std::move(gb), optInt(o, "block", fold ? 1024 : 512), optInt(o, "items", 4), {4}).launchBound =
+        1024;
     if (filter) {
-        ph.scalarParams = {"gb_val_cut"};
+        plan.phases.back().scalarParams = {"gb_val_cut"};
         plan.requiredScalars = {"gb_val_cut"};
+    }
+    if (fold) {
+        auto mg = std::make_unique<HipGroupByMerge>("d_gb_ht", "gb_slots", ldsSlots, pmax);
+        mg->setWindow(optInt(o, "window", 16));
+        auto& pm = appendPhase(plan, "GB_merge", std::move(mg), 1024, 16, {16});
+        pm.launchBound = 1024;
     }
     if (prepass) {
         plan.requiredScalars.push_back("gb_key_min");
@@ -518,8 +537,8 @@ HipQueryPlan buildPipeAgg(const PlanOptions& o) {
     gb->setWindow(optInt(o, "window", 4));  // measured best for the batched pipelines
     // partials=N: each block (work item) stores its LDS table as one of at
     // most min(N, rows / 16384 + 1) partial tables and PIPE_merge folds them
-    // into the table — one global merge per key and merge block instead of
-    // one per key and scan block
+    // into the table — one global merge per key instead of one per key and
+    // scan block
     const int partials = optInt(o, "partials", 0);
     const int cap = optInt(o, "lds_cap", 2048);
     const std::string pmax = "min(" + std::to_string(partials) + ", n_P / 16384 + 1)";
@@ -531,12 +550,9 @@ HipQueryPlan buildPipeAgg(const PlanOptions& o) {
     if (partials > 0) {
         auto mg = std::make_unique<HipGroupByMerge>("d_pipe_ht", "pipe_slots", cap, pmax);
         mg->setRuntimeLdsBits("pipe_lds_bits");
-        // a block folds ITEMS x block partial slots per tile (one 4096-slot
-        // partial at 256 x 16); at most 16 blocks, so a key is merged into
-        // the global table at most 16 times
+        mg->setWindow(optInt(o, "window", 4));
         auto& pm = appendPhase(plan, "PIPE_merge", std::move(mg), 256, 16, {16});
         pm.launchBound = 1024;
-        pm.maxThreadgroups = 16;
     }
     plan.requiredScalars = {"pipe_date_lo", "pipe_date_hi", "pipe_flag", "pipe_lds_bits"};
     plan.requiredSymbols = {"pipe_slots"};

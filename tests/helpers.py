@@ -55,3 +55,14 @@ def served_expected(T: dict, kind: str, params: dict, max_a: int, threads: int =
         h = oracle.q13(T["S"], T["A"], max_a, params["w1"], params["w2"], threads=threads)
         return {k: [int(x) for x in v] for k, v in h.items()}
     raise ValueError(kind)
+
+
+def group_rows(G: dict) -> dict:
+    """key (unsigned), count, sum, min, max of every key of G, ascending: by
+    sorting, so sparse keys cost no memory (the oracle's array spans the key range)."""
+    k = G["g_key"].view(np.uint32).astype(np.int64)
+    order = np.argsort(k, kind="stable")
+    k, v = k[order], G["g_val"][order]
+    at = np.flatnonzero(np.concatenate([[True], k[1:] != k[:-1]]))
+    return {"key": k[at], "count": np.diff(np.append(at, k.size)), "sum": np.add.reduceat(v, at),
+            "min": np.minimum.reduceat(v, at), "max": np.maximum.reduceat(v, at)}

@@ -1,0 +1,81 @@
+"""The LDS group-by's fold phase (partial tables -> group table): against a
+sort where it can go wrong — few blocks (no partials), LDS tables smaller
+than the groups (spills, keys probing past their home slot and round the
+table's end), tables filled over several runs or chunks, and as work items of
+a batch."""
+
+import numpy as np
+import pytest
+
+from gpudbmetalcodegen_amd import batch as B
+from gpudbmetalcodegen_amd import engine as E
+from gpudbmetalcodegen_amd import queries as Q
+from helpers import group_rows
+
+pytestmark = pytest.mark.gpu
+
+
+def _table(n, groups, seed, skew=False):
+    r = np.random.default_rng(seed)
+    k = r.integers(0, groups, n) if not skew else np.minimum(r.zipf(1.3, n), groups) - 1
+    return {"g_key": ((k * 2654435761) % (1 << 31)).astype(np.int32), "g_val": r.integers(-10**9, 10**9, n)}
+
+
+def _same(cols, G, times=1):
+    for c, e in group_rows(G).items():
+        assert np.array_equal(cols[c], e * (times if c in ("count", "sum") else 1)), c
+
+
+# rows: below and above 16 blocks of 2,048; groups: far below, at and above the LDS slots
+@pytest.mark.parametrize("lds_slots", [64, 1024, 4096])
+@pytest.mark.parametrize("n,groups", [(1, 1), (30_000, 500), (40_000, 500), (300_001, 60), (300_001, 1000), (300_001, 5000)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_fold_matches_oracle(ctx, lds_slots, n, groups, skew):
+    print(lds_slots, n, groups, skew, flush=True)
+    G = _table(n, groups, n + lds_slots, skew)
+    dev = Q.upload_tables(ctx, {"G": G})
+    try:
+        run = Q.run_groupby(ctx, dev, slots=2 * groups, variant="lds", lds_slots=lds_slots)
+        _same(run.result.columns, G)
+        run.executor.execute(run.plan, 1, 2)
+        _same(run.executor.collect(run.plan).columns, G)
+        # two runs into one table: the second folds only its own partials
+        run.executor.execute(run.plan)
+        run.executor.set_skip_init(True)
+        run.executor.execute(run.plan)
+        _same(run.executor.collect(run.plan).columns, G, times=2)
+    finally:
+        dev["G"].free(ctx)
+
+
+def test_fold_of_a_chunked_run(ctx):
+    G = _table(500_000, 700, 5)
+    h = E.HostTable("G", G)
+    try:
+        for chunk in (100_000, 4096, 500_000):   # more partials than there is room for, one, and none left over
+            run = Q.run_groupby(ctx, {}, slots=2048, variant="lds", stream=Q.Stream(h, chunk))
+            _same(run.result.columns, G)
+    finally:
+        h.close()
+
+
+@pytest.mark.parametrize("chunk", [2048, 20_000, 1 << 20])
+@pytest.mark.parametrize("lds_bits", [5, 9, 12])
+def test_fold_of_batched_pipelines(ctx, chunk, lds_bits):
+    specs = B.workload3(n_pipes=8, scale=0.05, seed=77)
+    w = B.Workload3(ctx, specs, lds_cap=4096, partials=32)
+    try:
+        w.run_plain()
+        plain = w.results()
+        for s in w.specs:
+            w.batch_launch[s.index] = (256, 4, lds_bits)
+        b = w.build_batch(512, 16_384, fold_rows=chunk)
+        try:
+            for _ in range(3):
+                b.run(graph=True)
+                for got, exp in zip(w.results(), plain):
+                    assert all(np.array_equal(got[k], exp[k]) for k in exp)
+        finally:
+            b.close()
+    finally:
+        w.close()
