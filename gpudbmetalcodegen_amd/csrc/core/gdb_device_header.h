@@ -278,7 +278,6 @@ GDB_DEV i64 gdb_ht_insert_unique(u64* __restrict__ tab, u32 slot_words, u32 bits
     const u64 mine = (u64)key | ((u64)payload << 32);
     // CAS first: at the load factors used (<= 1/2) the home slot is usually
     // empty, and a failed CAS returns the occupant, so no separate load.
-#pragma unroll 1
     for (u32 p = 0; p < max_probe; ++p, s = (s + 1) & mask) {
         u64* w = tab + s * slot_words;
         u64 cur = GDB_EMPTY_WORD;
@@ -296,7 +295,6 @@ GDB_DEV i64 gdb_ht_insert_unique(u64* __restrict__ tab, u32 slot_words, u32 bits
 GDB_DEV i64 gdb_ht_find(const u64* __restrict__ tab, u32 slot_words, u32 bits, u32 key, u32 max_probe) {
     const u64 mask = (1ull << bits) - 1ull;
     u64 s = gdb_hash_slot(key, bits);
-#pragma unroll 1
     for (u32 p = 0; p < max_probe; ++p, s = (s + 1) & mask) {
         const u32 k = (u32)tab[s * slot_words];
         if (k == key) return (i64)s;
@@ -325,7 +323,6 @@ GDB_DEV u64 gdb_hash_slot64(u64 key, u32 bits) { return (key * 0x9E3779B97F4A7C1
 GDB_DEV int gdb_ht64_insert_at(u64* __restrict__ tab, u32 bits, u64 key, u64 payload, u32 max_probe, i64* slot) {
     const u64 mask = (1ull << bits) - 1ull;
     u64 s = gdb_hash_slot64(key, bits);
-#pragma unroll 1
     for (u32 p = 0; p < max_probe; ++p, s = (s + 1) & mask) {
         const u64 seen = tab[2 * s];
         if (seen == key) {
@@ -375,7 +372,6 @@ GDB_DEV int gdb_ht64_insert(u64* __restrict__ tab, u32 bits, u64 key, u64 payloa
 GDB_DEV i64 gdb_ht64_find(const u64* __restrict__ tab, u32 bits, u64 key, u32 max_probe) {
     const u64 mask = (1ull << bits) - 1ull;
     u64 s = gdb_hash_slot64(key, bits);
-#pragma unroll 1
     for (u32 p = 0; p < max_probe; ++p, s = (s + 1) & mask) {
         const u64 k = tab[2 * s];
         if (k == key) return (i64)s;
@@ -391,7 +387,6 @@ GDB_DEV int gdb_gb_merge(u64* __restrict__ tab, u32 bits, u32 key, u32 cnt, i64 
                          u32 max_probe) {
     const u64 mask = (1ull << bits) - 1ull;
     u64 s = gdb_hash_slot(key, bits);
-#pragma unroll 1
     for (u32 p = 0; p < max_probe; ++p, s = (s + 1) & mask) {
         u64* w = tab + s * 4;
         u64 cur = gdb_load_relaxed_u64(w);
@@ -420,13 +415,16 @@ GDB_DEV int gdb_gb_merge(u64* __restrict__ tab, u32 bits, u32 key, u32 cnt, i64 
 // tab[j * slots + s] — so a wave's 64 random slots spread over 32 bank pairs
 // instead of the 8 a 32-byte slot-major layout reaches (measured ~8 conflict
 // cycles per LDS instruction with it). Returns the slot index, or -1 when the
-// probe window is full (caller spills to global). Probe loops stay rolled:
-// unrolled 16 times for each of a thread's rows they filled the instruction
-// cache (GB_agg of 100M rows: 502 -> 454 us rolled).
+// probe window is full (caller spills to global). U: the probe loop's unroll
+// count, 1 for wide windows — unrolled 16 times for each of a thread's rows
+// the code filled the instruction cache (GB_agg of 100M rows: 502 us, 454 us
+// rolled) — and the window itself up to 4 (GBP_count_flags of 40M rows at
+// window 2: 264 us rolled, 237 us unrolled).
+template <int U>
 GDB_DEV int gdb_lds_gb_update(u64* tab, u32 bits, u32 key, i64 v, u32 max_probe) {
     const u32 n = 1u << bits, mask = n - 1u;
     u32 s = (u32)gdb_hash_slot(key, bits);
-#pragma unroll 1
+#pragma unroll U
     for (u32 p = 0; p < max_probe; ++p, s = (s + 1) & mask) {
         u64* w = tab + s;
         u64 cur = gdb_lds_load_u64(w);
@@ -456,7 +454,7 @@ GDB_DEV int gdb_lds_gb_update(u64* tab, u32 bits, u32 key, i64 v, u32 max_probe)
 
 // Merge a partial group (cnt rows, sum/min/max) into a word-major LDS table
 // of (mask + 1) slots starting at slot s. Returns the slot or -1 after
-// max_probe slots.
+// max_probe slots (probe loop rolled, as above).
 GDB_DEV int gdb_lds_gb_merge_at(u64* tab, u32 mask, u32 s, u32 key, u32 cnt, i64 sum, i64 mn, i64 mx, u32 max_probe) {
     const u32 n = mask + 1u;
 #pragma unroll 1
@@ -488,7 +486,6 @@ GDB_DEV int gdb_lds_gb_merge_at(u64* tab, u32 mask, u32 s, u32 key, u32 cnt, i64
 GDB_DEV bool gdb_lds_key_member(const u32* keys, u32 bits, u32 key, u32 max_probe) {
     const u32 mask = (1u << bits) - 1u;
     u32 s = (u32)gdb_hash_slot(key, bits);
-#pragma unroll 1
     for (u32 p = 0; p < max_probe; ++p, s = (s + 1) & mask) {
         const u32 k = keys[s];
         if (k == key) return true;

@@ -1710,6 +1710,9 @@ std::pair<std::string, std::string> ldsTableSize(HipCodegen& cg, const std::stri
     return {"_ls_" + T, "_lb_" + T};
 }
 
+// Unroll count of gdb_lds_gb_update's probe loop for a probe window.
+int probeUnroll(int window) { return window <= 4 ? window : 1; }
+
 // Word-major LDS group table (word j of slot s at j * LS + s): empty slots.
 void emitLdsGbInit(HipCodegen& cg, const std::string& tab, const std::string& LS) {
     cg.addBlock("for (int _s = (int)threadIdx.x; _s < " + LS + "; _s += (int)blockDim.x)", [&]() {
@@ -1775,7 +1778,7 @@ void HipHashGroupBy::produceImpl(HipCodegen& cg, ConsumerFn consume) {
         child_->produce(cg, [&]() {
             cg.addLine("const u32 _gk = (u32)(" + key_ + ");");
             cg.addLine("const i64 _gv = (i64)(" + value_ + ");");
-            cg.addBlock("if (gdb_lds_gb_update(" + tab + ", " + LB + ", _gk, _gv, " + s(window_) + "u) < 0)", [&]() {
+            cg.addBlock("if (gdb_lds_gb_update<" + s(probeUnroll(window_)) + ">(" + tab + ", " + LB + ", _gk, _gv, " + s(window_) + "u) < 0)", [&]() {
                 cg.addLine("const int _r = " + merge1 + ";");
                 cg.addLine("if (_r < 0) ++_ovf_" + T + "; else _ins_" + T + " += (u32)_r;");
                 cg.addLine("++_spill_" + T + ";");
@@ -2079,7 +2082,7 @@ void HipPartitionCount::produceImpl(HipCodegen& cg, ConsumerFn consume) {
     child_->produce(cg, [&]() {
         cg.addLine("const u32 _gk = (u32)(" + key_ + ");");
         cg.addLine("const i64 _gv = (i64)(" + value_ + ");");
-        cg.addBlock("if (gdb_lds_gb_update(_gl, " + s(lbits) + "u, _gk, _gv, " + s(c_.window) + "u) < 0)", [&]() {
+        cg.addBlock("if (gdb_lds_gb_update<" + s(probeUnroll(c_.window)) + ">(_gl, " + s(lbits) + "u, _gk, _gv, " + s(c_.window) + "u) < 0)", [&]() {
             cg.addLine("gdb_lds_add_u32(&_pc[gdb_partition(_gk, _pb)], 1u);");
             cg.addLine("++_spill;");
             if (flags) setFlag("_gk");
@@ -2128,46 +2131,75 @@ void HipPartitionOffsets::produceImpl(HipCodegen& cg, ConsumerFn consume) {
     cg.addBufferParam(st, "u64", 8, "4", InitKind::Zero, {}, false, true);
     cg.setPhaseStatusBuffer(st);
     const std::string LB = s(PartitionConfig::kLogicalBlocks);
-    cg.setPhaseRowsExpr("(" + n.P + ") * 64");
+    // a block per 64 lanes of count partitions
+    cg.setPhaseRowsExpr("(" + n.PC + ") * 16");
     cg.addComment("counts -> exclusive offsets over the logical blocks, per partition, and totals; a partition's "
-                  "count is the sum of its consecutive count partitions");
+                  "count is the sum of its _f consecutive count partitions");
     cg.addLine("const u64 _P = " + n.NP + ", _PC = " + n.NPC + ";");
     cg.addLine("const bool _ok = _P <= _PC && _P <= " + s(c_.maxParts()) + "ull;");
-    cg.addLine("const u64 _f = _ok ? _PC / _P : 1;");
-    cg.addLine("const u64 _gt = (u64)blockIdx.x * blockDim.x + threadIdx.x, _nt = (u64)gridDim.x * blockDim.x;");
     cg.addBlock("if (!_ok)", [&]() {
         cg.addComment("more table partitions than count partitions or LDS counters: [0]+[1], and zero offsets "
                       "and totals, so the later passes of this (failed) run stay within their buffers");
+        cg.addLine("const u64 _gt = (u64)blockIdx.x * blockDim.x + threadIdx.x, _nt = (u64)gridDim.x * blockDim.x;");
         cg.addLine("if (_gt == 0) { gdb_atomic_max_u64(" + st + " + 0, 1ull); gdb_atomic_max_u64(" + st + " + 1, 1ull); }");
         cg.addLine("for (u64 _i = _gt; _i < " + LB + " * _P; _i += _nt) { " + n.coff + "[_i] = 0; " + n.poff + "[_i] = 0; }");
         cg.addLine("for (u64 _i = _gt; _i < 2 * _P; _i += _nt) " + n.meta + "[_i] = 0;");
     });
-    cg.addBlock("if (_f == 1)", [&]() {
-        cg.addComment("one thread per partition: consecutive lanes read consecutive counters");
-        cg.addBlock("for (u64 _q = _gt; _ok && _q < _P; _q += _nt)", [&]() {
-            cg.addLine("u32 _c = 0, _r = 0;");
-            cg.addBlock("for (u64 _lb = 0; _lb < " + LB + "; ++_lb)", [&]() {
-                cg.addLine("const u32 _a = " + n.ccnt + "[_lb * _PC + _q], _b = " + n.pcnt + "[_lb * _PC + _q];");
-                cg.addLine(n.coff + "[_lb * _P + _q] = _c; " + n.poff + "[_lb * _P + _q] = _r;");
-                cg.addLine("_c += _a; _r += _b;");
+    // Bound by latency: 8 MB of counts at most, but a serial walk over 256
+    // logical blocks per partition took 223 us (4,096 count partitions). Here
+    // 16 logical blocks' counts are in flight at once and a block's waves,
+    // 16 logical blocks each, meet in LDS: 7.5 us.
+    cg.addBlock("if (_ok)", [&]() {
+        static_assert(PartitionConfig::kLogicalBlocks == 256, "16 chunks of 16 logical blocks");
+        cg.addComment("_g lanes share a partition's count partitions; a block holds _q partitions");
+        cg.addLine("const u32 _f = (u32)(_PC / _P), _g = _f < 64u ? _f : 64u, _q = 64u / _g;");
+        cg.addLine("const u32 _ln = (u32)gdb_lane(), _nw = blockDim.x >> 6, _sub = _ln & (_g - 1u);");
+        cg.declareLds("u32", "_sc", "16 * 64");
+        cg.declareLds("u32", "_sp", "16 * 64");
+        cg.addBlock("for (u64 _q0 = (u64)blockIdx.x * _q; _q0 < _P; _q0 += (u64)gridDim.x * _q)", [&]() {
+            cg.addLine("const u64 _p = _q0 + _ln / _g;");
+            cg.addLine("const bool _have = _p < _P;");
+            cg.addLine("u32 _a[16], _b[16];");
+            cg.addComment("the 16 logical blocks of chunk _ch: this partition's counts, as exclusive sums in the chunk");
+            cg.addLine("u32 _c, _r;");
+            cg.addBlock("auto _chunk = [&](u32 _ch)", [&]() {
+                cg.addLine("const u64 _at = (u64)_ch * 16 * _PC + (_have ? _p : 0) * _f + _sub;");
+                cg.addLine("#pragma unroll");
+                cg.addLine("for (int _k = 0; _k < 16; ++_k) { _a[_k] = " + n.ccnt + "[_at + (u64)_k * _PC]; _b[_k] = " + n.pcnt +
+                           "[_at + (u64)_k * _PC]; }");
+                cg.addBlock("for (u32 _j = _g; _j < _f; _j += _g)", [&]() {
+                    cg.addLine("#pragma unroll");
+                    cg.addLine("for (int _k = 0; _k < 16; ++_k) { _a[_k] += " + n.ccnt + "[_at + _j + (u64)_k * _PC]; _b[_k] += " +
+                               n.pcnt + "[_at + _j + (u64)_k * _PC]; }");
+                });
+                cg.addBlock("for (u32 _d = 1; _d < _g; _d <<= 1)", [&]() {
+                    cg.addLine("#pragma unroll");
+                    cg.addLine("for (int _k = 0; _k < 16; ++_k) { _a[_k] += (u32)__shfl_xor((int)_a[_k], (int)_d, 64); _b[_k] += "
+                               "(u32)__shfl_xor((int)_b[_k], (int)_d, 64); }");
+                });
+                cg.addLine("_c = 0; _r = 0;");
+                cg.addLine("#pragma unroll");
+                cg.addLine("for (int _k = 0; _k < 16; ++_k) { const u32 _x = _a[_k], _y = _b[_k]; _a[_k] = _c; _b[_k] = _r; _c += _x; _r += _y; }");
+            }, ";");
+            cg.addLine("for (u32 _ch = (u32)gdb_wave(); _ch < 16u; _ch += _nw) { _chunk(_ch); _sc[_ch * 64u + _ln] = _c; _sp[_ch * 64u + _ln] = _r; }");
+            cg.addLine("__syncthreads();");
+            cg.addBlock("for (u32 _ch = (u32)gdb_wave(); _ch < 16u; _ch += _nw)", [&]() {
+                cg.addLine("if (_nw < 16u) _chunk(_ch);  // a full block still has it");
+                cg.addLine("u32 _cb = 0, _rb2 = 0, _ct = 0, _rt = 0;");
+                cg.addBlock("for (u32 _w = 0; _w < 16u; ++_w)", [&]() {
+                    cg.addLine("if (_w == _ch) { _cb = _ct; _rb2 = _rt; }");
+                    cg.addLine("_ct += _sc[_w * 64u + _ln]; _rt += _sp[_w * 64u + _ln];");
+                });
+                cg.addBlock("if (_have && _sub == 0)", [&]() {
+                    cg.addLine("#pragma unroll");
+                    cg.addBlock("for (int _k = 0; _k < 16; ++_k)", [&]() {
+                        cg.addLine("const u64 _o = ((u64)_ch * 16 + _k) * _P + _p;");
+                        cg.addLine(n.coff + "[_o] = _cb + _a[_k]; " + n.poff + "[_o] = _rb2 + _b[_k];");
+                    });
+                    cg.addLine("if (_ch == 0) { " + n.meta + "[_p] = _ct; " + n.meta + "[_P + _p] = _rt; }");
+                });
             });
-            cg.addLine(n.meta + "[_q] = _c; " + n.meta + "[_P + _q] = _r;");
-        });
-    });
-    cg.addBlock("else", [&]() {
-        cg.addComment("one wave per partition: the lanes sum its count partitions");
-        cg.addLine("const u64 _lane = threadIdx.x & 63u;");
-        cg.addBlock("for (u64 _q = _gt >> 6; _ok && _q < _P; _q += _nt >> 6)", [&]() {
-            cg.addLine("u64 _c = 0, _r = 0;");
-            cg.addBlock("for (u64 _lb = 0; _lb < " + LB + "; ++_lb)", [&]() {
-                cg.addLine("u64 _a = 0, _b = 0;");
-                cg.addLine("for (u64 _j = _lane; _j < _f; _j += 64) { _a += " + n.ccnt + "[_lb * _PC + _q * _f + _j]; _b += " +
-                           n.pcnt + "[_lb * _PC + _q * _f + _j]; }");
-                cg.addLine("_a = gdb_wave_sum_u64(_a); _b = gdb_wave_sum_u64(_b);");
-                cg.addLine("if (_lane == 0) { " + n.coff + "[_lb * _P + _q] = (u32)_c; " + n.poff + "[_lb * _P + _q] = (u32)_r; }");
-                cg.addLine("_c += _a; _r += _b;");
-            });
-            cg.addLine("if (_lane == 0) { " + n.meta + "[_q] = (u32)_c; " + n.meta + "[_P + _q] = (u32)_r; }");
+            cg.addLine("__syncthreads();");
         });
     });
     consume();

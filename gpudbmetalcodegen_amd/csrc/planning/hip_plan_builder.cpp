@@ -338,8 +338,8 @@ HipQueryPlan buildGroupBy(const PlanOptions& o) {
             gbCountFlagsPhase(plan);
             plan.sizingRules.push_back(sizing);
         }
-        auto& p2 = appendPhase(plan, "GBP_offsets", std::make_unique<HipPartitionOffsets>(pc), 256, 1, {1});
-        p2.launchBound = 256;
+        auto& p2 = appendPhase(plan, "GBP_offsets", std::make_unique<HipPartitionOffsets>(pc), 1024, 1, {1});
+        p2.launchBound = 1024;
         auto& p3 = appendPhase(plan, "GBP_bases", std::make_unique<HipPartitionBases>(pc), 1024, 1, {1});
         p3.launchBound = 1024;
         // pass 4 re-reads the rows (same scan, same filter)
