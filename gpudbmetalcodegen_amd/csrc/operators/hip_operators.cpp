@@ -774,9 +774,12 @@ void HipLikeFilter::produceImpl(HipCodegen& cg, ConsumerFn consume) {
     cg.addLine("gdb_like2_tables(" + t1 + ", " + t2 + ", (const char*)" + words_ + ", (int)" + l1_ + ", (const char*)" +
                words_ + " + 32, (int)" + l2_ + ");");
     cg.addLine("__syncthreads();");
+    const std::string h1 = t1 + "_h", h2 = t2 + "_h";
+    const std::string a1 = "(const char*)" + words_ + ", (int)" + l1_, a2 = "(const char*)" + words_ + " + 32, (int)" + l2_;
+    cg.addLine("const GdbLikeWord " + h1 + " = gdb_like_word(" + a1 + "), " + h2 + " = gdb_like_word(" + a2 + ");");
     child_->produce(cg, [&]() {
-        cg.addIf(std::string(negate_ ? "!" : "") + "gdb_like2_bp<" + s(width_) + ">(" + column_ + ", " + t1 + ", " + t2 +
-                     ", (int)" + l1_ + ", (int)" + l2_ + ")",
+        cg.addIf(std::string(negate_ ? "!" : "") + "gdb_like2_heads<" + s(width_) + ">(" + column_ + ", " + t1 + ", " + t2 +
+                     ", " + a1 + ", " + h1 + ", " + a2 + ", " + h2 + ")",
                  [&]() { consume(); });
     });
 }
@@ -1635,13 +1638,24 @@ void HipAtomicCount::produceImpl(HipCodegen& cg, ConsumerFn consume) {
         const std::string S = s(static_);
         cg.addComment("AtomicCount " + array_ + ": LDS histogram of " + S + " bins");
         cg.declareLds("u32", "_hist_" + array_, S);
+        // The first bins are counted in registers: histograms of counts have
+        // most rows in bins 0..3, on whose LDS atomics all lanes would meet.
+        const int regs = std::min(4, static_);
+        cg.addLine("u32 _hr_" + array_ + "[" + s(regs) + "] = {};");
         cg.addLine("for (int _h = (int)threadIdx.x; _h < " + S + "; _h += (int)blockDim.x) _hist_" + array_ + "[_h] = 0;");
         cg.addLine("__syncthreads();");
         child_->produce(cg, [&]() {
             cg.addLine("const u64 _hb = (u64)(i64)(" + bucket_ + ");");
-            cg.addLine("if (_hb < " + S + "ull && _hb < nelem_" + array_ + ") gdb_lds_add_u32(&_hist_" + array_ +
+            cg.addLine("#pragma unroll");
+            cg.addLine("for (int _h = 0; _h < " + s(regs) + "; ++_h) _hr_" + array_ + "[_h] += _hb == (u64)_h ? 1u : 0u;");
+            cg.addLine("if (_hb >= " + s(regs) + "ull && _hb < " + S + "ull && _hb < nelem_" + array_ + ") gdb_lds_add_u32(&_hist_" + array_ +
                        "[_hb], 1u);");
             consume();
+        });
+        cg.addLine("#pragma unroll");
+        cg.addBlock("for (int _h = 0; _h < " + s(regs) + "; ++_h)", [&]() {
+            cg.addLine("const u32 _n = (u32)gdb_wave_sum_u64((u64)_hr_" + array_ + "[_h]);");
+            cg.addLine("if (gdb_lane() == 0 && _n && (u64)_h < nelem_" + array_ + ") gdb_lds_add_u32(&_hist_" + array_ + "[_h], _n);");
         });
         cg.addLine("__syncthreads();");
         cg.addLine("for (int _h = (int)threadIdx.x; _h < " + S + "; _h += (int)blockDim.x) if ((u64)_h < nelem_" +
