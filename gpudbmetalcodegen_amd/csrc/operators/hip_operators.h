@@ -411,10 +411,11 @@ private:
 
 // LIKE '%w1%w2%' (NOT LIKE with negate) on a char[width] column staged in
 // LDS, byte-exact (q13_comment_match, metal_plan_builder.cpp:1249-1266, for
-// any two words): bit-parallel Shift-And automata over the row with per-block
-// LDS byte tables built from the words buffer (w1 at byte 0, w2 at byte 32;
-// lengths in two scalars). The phase must register the words buffer and the
-// length scalars.
+// any two words): both words' first four bytes against every window of the
+// row, and for rows that does not settle bit-parallel Shift-And automata with
+// per-block LDS byte tables built from the words buffer (w1 at byte 0, w2 at
+// byte 32; lengths in two scalars). The phase must register the words buffer
+// and the length scalars.
 class HipLikeFilter : public HipUnaryOperator {
 public:
     HipLikeFilter(std::unique_ptr<HipOperator> child, const std::string& column, int width,

@@ -95,7 +95,8 @@ class ResidentDB:
         if q.kind == "scan":
             return 4096
         if q.kind == "anti":
-            return self.max_a // 8 + 4096
+            flags = Q.q22_flags(self.n["B"], self.max_a + 1)
+            return self.max_a // 8 + (self.max_a + 1 if flags else 0) + 4096
         if q.kind == "like":
             return 4 * (self.max_a + 1) + 8192
         # join: A/B bitmaps + a hash table for the qualifying B rows, with

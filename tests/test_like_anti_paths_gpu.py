@@ -42,3 +42,28 @@ def test_like_small_alphabets(ctx, alphabet, n):
     finally:
         for t in dev.values():
             t.free(ctx)
+
+
+@pytest.mark.parametrize("n_a,n_b", [(31, 1000), (32, 1), (4095, 70_001), (100_003, 1_000_003)])
+def test_anti_join_by_flags_equals_bitmap(ctx, n_a, n_b, monkeypatch):
+    """Referenced keys as packed byte flags: key ranges around whole bitmap
+    words, keys outside the range, and no referencing row at all."""
+    r = np.random.default_rng(n_a)
+    A = {"a_key": (r.permutation(n_a) + 1).astype(np.int32), "a_seg": r.integers(0, 5, n_a).astype(np.uint8)}
+    B = {"b_key": np.arange(1, n_b + 1, dtype=np.int32), "b_fkey": r.integers(-3, n_a + 40, n_b).astype(np.int32),
+         "b_date": r.integers(0, 2406, n_b).astype(np.int32)}
+    dev = Q.upload_tables(ctx, {"A": A, "B": B})
+    try:
+        for lo, hi in [(0, 2406), (100, 300), (7, 7)]:
+            monkeypatch.setattr(Q, "Q22_FLAG_ROWS", 1 << 40)
+            plain = Q.run_q22(ctx, dev, lo, hi)
+            monkeypatch.setattr(Q, "Q22_FLAG_ROWS", 0)
+            flags = Q.run_q22(ctx, dev, lo, hi)
+            assert "Q22_pack_bitmap" in flags.plan.phases() and "Q22_pack_bitmap" not in plain.plan.phases()
+            assert flags.result.canonical == plain.result.canonical
+            hit = np.isin(A["a_key"], B["b_fkey"][(B["b_date"] >= lo) & (B["b_date"] < hi)])
+            assert int(np.sum(flags.result.columns["num_keys"])) == int((~hit).sum())
+            assert int(np.sum(flags.result.columns["sum_keys"])) == int(A["a_key"][~hit].astype(np.int64).sum())
+    finally:
+        for t in dev.values():
+            t.free(ctx)
