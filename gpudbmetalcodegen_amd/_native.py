@@ -190,6 +190,8 @@ def load() -> tuple[C.CDLL, C.CDLL]:
     _sig(eng, "gdb_result_str", [vp, i32, vp, sz])
     _sig(eng, "gdb_result_column_format", [vp, i32, P(i32), P(i32)])
     _sig(eng, "gdb_result_canonical", [vp, vp, sz, P(sz)])
+    _sig(eng, "gdb_result_describe", [vp, cstr, sz, P(sz)])
+    _sig(eng, "gdb_result_words", [vp, vp])
     # TPC-H ingest and the golden check
     _sig(eng, "gdb_tpch_column", [cstr, cstr, P(i32), P(i32), P(i32)])
     _sig(eng, "gdb_tpch_table_columns", [cstr, vp, sz, P(sz)])
@@ -251,9 +253,17 @@ def eng_check(st: int) -> None:
         raise (GdbOverflow if st == GDB_ERR_OVERFLOW else GdbError)(st, msg)
 
 
-def two_call_string(fn, *args) -> str:
+def two_call_string(fn, *args, guess: int = 0) -> str:
+    """A string the library returns by size, then by content; with a guess of
+    its size usually in one call."""
     need = sz(0)
-    eng_check(fn(*args, None, 0, C.byref(need)))
+    if guess:
+        buf = C.create_string_buffer(guess)
+        eng_check(fn(*args, buf, guess, C.byref(need)))
+        if need.value <= guess:
+            return buf.value.decode()
+    else:
+        eng_check(fn(*args, None, 0, C.byref(need)))
     buf = C.create_string_buffer(need.value)
     eng_check(fn(*args, buf, need.value, C.byref(need)))
     return buf.value.decode()

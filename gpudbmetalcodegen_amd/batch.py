@@ -250,7 +250,7 @@ class Workload3:
     def results(self) -> list[dict]:
         out = []
         for i, s in enumerate(self.specs):
-            res = self.execs[i].collect(self.plans[s.kind])
+            res = self.execs[i].collect(self.plans[s.kind], canonical=False)
             out.append({k: np.asarray(v) for k, v in res.columns.items()})
         return out
 

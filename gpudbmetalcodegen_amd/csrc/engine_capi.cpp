@@ -99,6 +99,8 @@ struct gdb_executor_s {
 
 struct gdb_result_s {
     GenericResult r;
+    std::string text;  // the canonical CSV, once asked for
+    bool haveText = false;
 };
 
 extern "C" {
@@ -659,7 +661,46 @@ gdb_status gdb_result_str(gdb_result r, int idx, char* out, size_t width) {
 }
 
 gdb_status gdb_result_canonical(gdb_result r, char* buf, size_t cap, size_t* need) {
-    return guard([&]() -> gdb_status { return copyOut(r->r.toCanonical(), buf, cap, need); });
+    return guard([&]() -> gdb_status {
+        if (!r->haveText) {  // callers ask twice: for the size, then for the text
+            r->text = r->r.toCanonical();
+            r->haveText = true;
+        }
+        return copyOut(r->text, buf, cap, need);
+    });
+}
+
+gdb_status gdb_result_describe(gdb_result r, char* buf, size_t cap, size_t* need) {
+    return guard([&]() -> gdb_status {
+        std::string d = std::to_string(r->r.rows());
+        for (const auto& c : r->r.columns) {
+            d += '\x1e' + c.name + '\x1f' + std::to_string(static_cast<int>(c.type)) + '\x1f' + std::to_string(c.scale) +
+                 '\x1f' + (c.date ? '1' : '0');
+            bool plain = c.type == ResultColumn::STR;  // values with a separator are left to gdb_result_str
+            for (const auto& v : c.str) plain = plain && v.find_first_of("\x1e\x1f") == std::string::npos;
+            if (plain)
+                for (const auto& v : c.str) d += '\x1f' + v;
+        }
+        return copyOut(d, buf, cap, need);
+    });
+}
+
+gdb_status gdb_result_words(gdb_result r, int64_t* out) {
+    return guard([&]() -> gdb_status {
+        for (const auto& c : r->r.columns) {
+            if (c.type == ResultColumn::I64) {
+                c.copyI64(out);
+                out += c.size();
+            } else if (c.type == ResultColumn::I128) {
+                for (__int128 v : c.i128) {
+                    const unsigned __int128 u = static_cast<unsigned __int128>(v);
+                    *out++ = static_cast<int64_t>(static_cast<uint64_t>(u));
+                    *out++ = static_cast<int64_t>(static_cast<uint64_t>(u >> 64));
+                }
+            }
+        }
+        return GDB_OK;
+    });
 }
 
 gdb_status gdb_result_free(gdb_result r) {

@@ -157,6 +157,7 @@ class HipQueryPlan:
         self.compile_ms = 0.0
         self.cache_hit = False
         self.plan_hash = 0
+        self._phases = None
 
     @property
     def handle(self):
@@ -175,6 +176,8 @@ class HipQueryPlan:
         return json.loads(N.two_call_string(_eng().gdb_plan_sql_layout, self._h))
 
     def phases(self) -> list[str]:
+        if self._phases is not None:
+            return list(self._phases)
         n = C.c_int()
         N.eng_check(_eng().gdb_plan_phase_count(self._h, C.byref(n)))
         out = []
@@ -182,6 +185,7 @@ class HipQueryPlan:
             buf = C.create_string_buffer(256)
             N.eng_check(_eng().gdb_plan_phase_name(self._h, i, buf, 256))
             out.append(buf.value.decode())
+        self._phases = tuple(out)   # a built plan's phases do not change
         return out
 
     def set_launch(self, phase: str, block: int, items: int) -> None:
@@ -395,40 +399,57 @@ class HipGenericExecutor:
         N.eng_check(_eng().gdb_executor_owned_bytes(self._h, C.byref(n)))
         return n.value
 
-    def collect(self, plan: HipQueryPlan) -> GenericResult:
+    def collect(self, plan: HipQueryPlan, canonical: bool = True) -> GenericResult:
+        """The plan's result on the host; canonical=False leaves its CSV text
+        out (for callers that only take the columns)."""
+        eng = _eng()
         r = C.c_void_p()
-        N.eng_check(_eng().gdb_executor_collect(self._h, plan.handle, C.byref(r)))
+        N.eng_check(eng.gdb_executor_collect(self._h, plan.handle, C.byref(r)))
         try:
-            rows, cols = C.c_uint64(), C.c_int()
-            N.eng_check(_eng().gdb_result_shape(r, C.byref(rows), C.byref(cols)))
+            head = N.two_call_string(eng.gdb_result_describe, r, guess=4096).split("\x1e")
+            rows = int(head[0])
+            cols = [h.split("\x1f") for h in head[1:]]
             out, fmts = {}, {}
-            for i in range(cols.value):
-                name = C.create_string_buffer(128)
-                typ = C.c_int()
-                N.eng_check(_eng().gdb_result_column(r, i, name, 128, C.byref(typ)))
-                nm = name.value.decode()
-                if typ.value == 0:
-                    a = np.empty(rows.value, dtype=np.int64)
-                    N.eng_check(_eng().gdb_result_i64(r, i, a.ctypes.data_as(C.c_void_p)))
-                elif typ.value == 1:
-                    w = np.empty(2 * rows.value, dtype=np.int64)
-                    N.eng_check(_eng().gdb_result_i128(r, i, w.ctypes.data_as(C.c_void_p)))
-                    a = np.array([int(np.uint64(w[2 * k])) + (int(w[2 * k + 1]) << 64) for k in range(rows.value)],
-                                 dtype=object)
+            kinds = [int(c[1]) for c in cols]
+            words = None
+            if rows <= 65536:  # every numeric column with one call, as slices of one array
+                words = np.empty(rows * sum((1, 2, 0)[k] for k in kinds), dtype=np.int64)
+                N.eng_check(eng.gdb_result_words(r, words.ctypes.data))
+            at = 0
+            for i, (c, kind) in enumerate(zip(cols, kinds)):
+                n = rows * (1, 2, 0)[kind]
+                if kind == 0 and words is None:
+                    a = np.empty(rows, dtype=np.int64)
+                    N.eng_check(eng.gdb_result_i64(r, i, a.ctypes.data))
+                elif kind == 0:
+                    a = words[at:at + n]
+                elif kind == 1:
+                    if words is not None:
+                        w = words[at:at + n]
+                    else:
+                        w = np.empty(n, dtype=np.int64)
+                        N.eng_check(eng.gdb_result_i128(r, i, w.ctypes.data))
+                    w = w.tolist()
+                    a = np.array([(lo & 0xFFFFFFFFFFFFFFFF) + (hi << 64) for lo, hi in zip(w[::2], w[1::2])], dtype=object)
                 else:
-                    width = 64
-                    raw = C.create_string_buffer(width * max(1, rows.value))
-                    N.eng_check(_eng().gdb_result_str(r, i, raw, width))
-                    a = np.array([raw.raw[k * width:(k + 1) * width].rstrip(b"\0").decode() for k in range(rows.value)],
-                                 dtype=object)
-                out[nm] = a
-                sc, dt = C.c_int(), C.c_int()
-                N.eng_check(_eng().gdb_result_column_format(r, i, C.byref(sc), C.byref(dt)))
-                fmts[nm] = (sc.value, bool(dt.value))
-            canon = N.two_call_string(_eng().gdb_result_canonical, r) if rows.value <= 100000 else ""
+                    a = np.array(c[4:] if len(c) == 4 + rows else self._strings(r, i, rows), dtype=object)
+                at += n
+                out[c[0]] = a
+                fmts[c[0]] = (int(c[2]), c[3] == "1")
+            canon = ""
+            if canonical and rows <= 100000:
+                canon = N.two_call_string(eng.gdb_result_canonical, r, guess=256 + 16 * len(cols) * (rows + 1))
             return GenericResult(out, canon, fmts)
         finally:
-            _eng().gdb_result_free(r)
+            eng.gdb_result_free(r)
+
+    @staticmethod
+    def _strings(r, i: int, rows: int) -> list:
+        """A string column whose values hold the separators of the description."""
+        width = 64
+        raw = C.create_string_buffer(width * max(1, rows))
+        N.eng_check(_eng().gdb_result_str(r, i, raw, width))
+        return [raw.raw[k * width:(k + 1) * width].rstrip(b"\0").decode() for k in range(rows)]
 
     def release(self) -> None:
         N.eng_check(_eng().gdb_executor_release(self._h))

@@ -185,6 +185,13 @@ gdb_status gdb_result_column_format(gdb_result r, int idx, int* scale, int* is_d
  * ',' '"' or a line break (GenericResult::toCanonical,
  * metal_result_collector.cpp:85-122, which prints doubles with %.4f). */
 gdb_status gdb_result_canonical(gdb_result r, char* buf, size_t cap, size_t* need);
+/* The whole result in two calls: its rows and columns as one line of text
+ * (the row count; then per column, each after a 0x1E: name, type, scale,
+ * is_date and the values of a string column, separated by 0x1F), and the
+ * numeric columns one after another (rows words each, two per 128-bit value,
+ * low word first). */
+gdb_status gdb_result_describe(gdb_result r, char* buf, size_t cap, size_t* need);
+gdb_status gdb_result_words(gdb_result r, int64_t* out);
 gdb_status gdb_result_free(gdb_result r);
 
 /* ---- TPC-H ingest: .tbl -> .colbin v2, and the golden check ----

@@ -1,0 +1,71 @@
+"""A collected result against itself: the canonical CSV rendered again in
+Python from the columns and formats, over results with fixed-point, 128-bit,
+negative, date and string columns, extreme values, no rows, and labels that
+hold the separators of the one-call description."""
+
+import numpy as np
+import pytest
+
+from gpudbmetalcodegen_amd import queries as Q
+from gpudbmetalcodegen_amd import tpch as T
+from gpudbmetalcodegen_amd import tpch_gen as G
+from gpudbmetalcodegen_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _text(res) -> str:
+    lines = [",".join(res.columns)]
+    for r in range(res.rows()):
+        f = []
+        for name, col in res.columns.items():
+            scale, date = res.formats[name]
+            v = col[r]
+            if isinstance(v, str):
+                f.append('"' + v.replace('"', '""') + '"' if any(c in v for c in ',"\n\r') else v)
+            elif date:
+                f.append(f"{int(v) // 10000:04d}-{int(v) // 100 % 100:02d}-{int(v) % 100:02d}")
+            elif scale:
+                d = str(abs(int(v))).rjust(scale + 1, "0")
+                f.append(("-" if v < 0 else "") + d[:-scale] + "." + d[-scale:])
+            else:
+                f.append(str(int(v)))
+        lines.append(",".join(f))
+    return "\n".join(lines) + "\n"
+
+
+def test_named_plans_text(ctx):
+    db = T.TpchDB(ctx, G.generate(0.01, seed=3))
+    try:
+        for q in ("Q1", "Q3", "Q6", "Q10", "Q11", "Q13", "Q18", "Q21", "Q22"):
+            res = T.run(ctx, db, q).raw
+            assert res.canonical == _text(res), q
+        for label in ("M\x1fA", "M\x1eA", 'M"A'):
+            r = T.run(ctx, db, "Q12", options=f"mode1={label}")
+            assert r.raw.canonical == _text(r.raw) and label in list(next(iter(r.raw.columns.values())))
+    finally:
+        db.free()
+
+
+def test_scan_text_and_no_rows(ctx):
+    dev = Q.upload_tables(ctx, W.workload0(5000))
+    try:
+        for cutoff in (W.q1_cutoff(), -1):
+            res = Q.run_q1(ctx, dev, cutoff).result
+            assert res.canonical == _text(res) and res.rows() == (6 if cutoff >= 0 else 0)
+            assert all(v.dtype == (np.int64 if k.startswith(("sum_qty", "sum_base", "count")) else v.dtype)
+                       for k, v in res.columns.items())
+    finally:
+        dev["F"].free(ctx)
+
+
+def test_extreme_values_text(ctx):
+    lo, hi = -2**63, 2**63 - 1
+    G_ = {"g_key": np.array([1, 2, 3, 4, 4], np.int32), "g_val": np.array([lo, hi, 0, -1, 1], np.int64)}
+    dev = Q.upload_tables(ctx, {"G": G_})
+    try:
+        res = Q.run_groupby(ctx, dev, slots=64, variant="global").result
+        assert list(res.columns["min"]) == [lo, hi, 0, -1] and list(res.columns["max"]) == [lo, hi, 0, 1]
+        assert res.canonical == _text(res)
+    finally:
+        dev["G"].free(ctx)
