@@ -29,24 +29,39 @@ HipGenericExecutor::HipGenericExecutor(gdb_ctx ctx, gdb_stream stream)
 HipGenericExecutor::~HipGenericExecutor() {
     releaseAllocatedBuffers();
     for (auto e : events_) gdb_event_destroy(e);
-    if (dStatusPtrs_) gdb_free(ctx_, dStatusPtrs_);
-    if (dStatusOut_) gdb_free(ctx_, dStatusOut_);
-    if (pinned_) gdb_host_free_pinned(pinned_);
+    dropPinned();
 }
 
 uint64_t* HipGenericExecutor::ensurePinned(size_t bytes) {
     if (bytes > pinnedBytes_) {
         check(gdb_stream_sync(stream_), "gdb_stream_sync");  // no copy into the old block is in flight
-        if (pinned_) gdb_host_free_pinned(pinned_);
-        pinned_ = nullptr;
-        pinnedBytes_ = 0;
-        const size_t nb = std::max<size_t>(bytes, 8192);
+        pinnedInFlight_ = false;
+        dropPinned();
         void* h = nullptr;
-        check(gdb_host_alloc_pinned(nb, &h), "gdb_host_alloc_pinned");
+        if (bytes <= GDB_PINNED_BLOCK)
+            check(gdb_host_take_block(&h), "gdb_host_take_block");
+        else
+            check(gdb_host_alloc_pinned(bytes, &h), "gdb_host_alloc_pinned");
         pinned_ = static_cast<uint64_t*>(h);
-        pinnedBytes_ = nb;
+        pinnedBytes_ = std::max<size_t>(bytes, GDB_PINNED_BLOCK);
     }
+    pinnedInFlight_ = true;  // until the caller has waited for what it enqueues
     return pinned_;
+}
+
+void HipGenericExecutor::dropPinned() {
+    // a block something may still write (a failed run) is freed, which waits, and not shared again
+    if (pinnedBytes_ == GDB_PINNED_BLOCK && !pinnedInFlight_)
+        gdb_host_give_block(pinned_);
+    else if (pinned_)
+        gdb_host_free_pinned(pinned_);
+    pinned_ = nullptr;
+    pinnedBytes_ = 0;
+}
+
+void HipGenericExecutor::syncStream() {
+    check(gdb_stream_sync(stream_), "gdb_stream_sync");
+    pinnedInFlight_ = false;
 }
 
 void HipGenericExecutor::registerTable(const std::string& table, uint64_t rows) {
@@ -252,9 +267,10 @@ void HipGenericExecutor::prepare(const HipCodegen& cg, int firstPhase, int lastP
 void HipGenericExecutor::launchPhase(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq,
                                      const HipCodegen::PhaseInfo& p, std::unordered_map<std::string, bool>& initDone,
                                      const std::unordered_map<std::string, const HipParamBinding*>& initSpec,
-                                     unsigned* gridOut, gdb_event beforeKernel) {
+                                     unsigned* gridOut, gdb_event beforeKernel, bool* marked) {
     std::vector<uint64_t> args;
     args.reserve(p.bindings.size());
+    bool filled = false;
     resolveBufferTables();
     for (const auto& b : p.bindings) {
         switch (b.kind) {
@@ -295,6 +311,7 @@ void HipGenericExecutor::launchPhase(RuntimeCompiler& rc, const RuntimeCompiler:
                                                  stream_),
                                   "fill " + b.name);
                         }
+                        filled = true;
                         initDone[b.name] = true;
                     }
                 }
@@ -329,7 +346,13 @@ void HipGenericExecutor::launchPhase(RuntimeCompiler& rc, const RuntimeCompiler:
         grid = static_cast<unsigned>(std::min(need, cap));
     }
     if (gridOut) *gridOut = grid;
-    if (beforeKernel) check(gdb_event_record(beforeKernel, stream_), "gdb_event_record");
+    // A phase begins where the one before it ended unless something came
+    // between (fills; *marked set by the caller: the start of the run, a hook):
+    // a second event record between back-to-back kernels only cost time.
+    if (beforeKernel && (filled || *marked)) {
+        check(gdb_event_record(beforeKernel, stream_), "gdb_event_record");
+        *marked = true;
+    }
     check(gdb_launch(k, grid, static_cast<unsigned>(block), 0, args.data(), args.size() * 8, stream_),
           "launch " + p.name);
 }
@@ -432,7 +455,7 @@ void HipGenericExecutor::enqueue(RuntimeCompiler& rc, const RuntimeCompiler::Com
     std::unordered_map<std::string, bool> initDone;
     hoistInits(cg, firstPhase, last, initDone, spec);
     for (int pi = firstPhase; pi < last; ++pi)
-        launchPhase(rc, cq, phases[static_cast<size_t>(pi)], initDone, spec, nullptr);
+        launchPhase(rc, cq, phases[static_cast<size_t>(pi)], initDone, spec, nullptr, nullptr, nullptr);
 }
 
 HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq,
@@ -467,11 +490,16 @@ HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const Runtim
         res.phaseItems.clear();
         check(gdb_event_record(events_[0], stream_), "gdb_event_record");
         hoistInits(cg, firstPhase, last, initDone, spec);
+        bool apart = true;  // something lies between the last event recorded and the next phase
+        ownStart_.assign(static_cast<size_t>(np), true);
         for (int pi = firstPhase; pi < last; ++pi) {
             const auto& p = phases[static_cast<size_t>(pi)];
             unsigned grid = 0;
             const size_t e = static_cast<size_t>(2 * (pi - firstPhase));
-            launchPhase(rc, cq, p, initDone, spec, &grid, phaseTiming_ ? events_[e + 1] : nullptr);
+            bool marked = apart;
+            launchPhase(rc, cq, p, initDone, spec, &grid, phaseTiming_ ? events_[e + 1] : nullptr, &marked);
+            ownStart_[static_cast<size_t>(pi - firstPhase)] = marked;
+            apart = false;
             if (phaseTiming_ || pi + 1 == last) check(gdb_event_record(events_[e + 2], stream_), "gdb_event_record");
             res.phaseNames.push_back(p.name);
             res.phaseGrid.push_back(grid);
@@ -489,14 +517,15 @@ HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const Runtim
                                                h->second.bytes, stream_),
                           "hook read " + h->second.buffer);
                 }
-                check(gdb_stream_sync(stream_), "gdb_stream_sync");
+                syncStream();
                 h->second.fn(*this);
+                apart = true;
             }
         }
         if (r + 1 == runs) {
             // the final run: status words gathered and read behind it, one wait for both
             pending = enqueueStatus(cg, firstPhase, last);
-            check(gdb_stream_sync(stream_), "gdb_stream_sync");
+            syncStream();
         } else {
             check(gdb_event_sync(events_[static_cast<size_t>(2 * np)]), "gdb_event_sync");
         }
@@ -505,8 +534,9 @@ HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const Runtim
             for (int i = 0; phaseTiming_ && i < np; ++i) {
                 float ms = 0.0f, fill = 0.0f;
                 const size_t e = static_cast<size_t>(2 * i);
-                check(gdb_event_elapsed_ms(events_[e + 1], events_[e + 2], &ms), "gdb_event_elapsed_ms");
-                check(gdb_event_elapsed_ms(events_[e], events_[e + 1], &fill), "gdb_event_elapsed_ms");
+                const bool own = ownStart_[static_cast<size_t>(i)];
+                check(gdb_event_elapsed_ms(events_[own ? e + 1 : e], events_[e + 2], &ms), "gdb_event_elapsed_ms");
+                if (own) check(gdb_event_elapsed_ms(events_[e], events_[e + 1], &fill), "gdb_event_elapsed_ms");
                 measuredPhase_[static_cast<size_t>(i)] += ms * w;
                 measuredFill_[static_cast<size_t>(i)] += fill * w;
             }
@@ -523,48 +553,31 @@ HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const Runtim
 
 HipGenericExecutor::PendingStatus HipGenericExecutor::enqueueStatus(const HipCodegen& cg, int firstPhase,
                                                                     int lastPhase) {
-    // Every status and check word of the range is gathered on the device and
-    // read back with one copy; the caller's next synchronisation covers it.
+    // Every status and check word of the range is written to pinned memory by
+    // one launch; the caller's next synchronisation covers it.
     const auto& phases = cg.getPhases();
     const int last = lastPhase < 0 ? static_cast<int>(phases.size()) : lastPhase;
     PendingStatus ps;
     ps.phases = static_cast<size_t>(std::max(0, last - firstPhase));
-    std::vector<const void*> ptrs;
+    std::vector<gdb_gather_piece> pieces;
+    auto add = [&](int phase, void* words, const std::string& name, bool isCheck, const std::string& message) {
+        pieces.push_back({words, 32u, static_cast<uint32_t>(32 * pieces.size())});
+        ps.refs.push_back({phase, {words, name, isCheck, message}});
+    };
     for (int pi = firstPhase; pi < last; ++pi) {
         const auto& p = phases[static_cast<size_t>(pi)];
         auto st = buffers_.find(p.statusBuffer);
-        if (!p.statusBuffer.empty() && st != buffers_.end()) {
-            ps.refs.push_back({pi - firstPhase, {st->second.ptr, p.name, false, ""}});
-            ptrs.push_back(st->second.ptr);
-        }
+        if (!p.statusBuffer.empty() && st != buffers_.end()) add(pi - firstPhase, st->second.ptr, p.name, false, "");
         auto ck = buffers_.find(p.checkBuffer);
-        if (!p.checkBuffer.empty() && ck != buffers_.end()) {
-            ps.refs.push_back({pi - firstPhase, {ck->second.ptr, p.name, true, p.checkMessage}});
-            ptrs.push_back(ck->second.ptr);
-        }
+        if (!p.checkBuffer.empty() && ck != buffers_.end())
+            add(pi - firstPhase, ck->second.ptr, p.name, true, p.checkMessage);
     }
     if (ps.refs.empty()) return ps;
-    const size_t n = ps.refs.size();
-    uint64_t* host = ensurePinned(n * 32 + n * sizeof(void*));
-    if (n > statusCap_) {
-        check(gdb_stream_sync(stream_), "gdb_stream_sync");
-        if (dStatusPtrs_) gdb_free(ctx_, dStatusPtrs_);
-        if (dStatusOut_) gdb_free(ctx_, dStatusOut_);
-        dStatusPtrs_ = dStatusOut_ = nullptr;
-        statusCap_ = std::max<size_t>(n, 64);
-        check(gdb_alloc(ctx_, statusCap_ * sizeof(void*), &dStatusPtrs_), "gdb_alloc");
-        check(gdb_alloc(ctx_, statusCap_ * 32, &dStatusOut_), "gdb_alloc");
-        statusPtrCache_.clear();
-    }
-    if (ptrs != statusPtrCache_) {
-        std::memcpy(host + 4 * n, ptrs.data(), n * sizeof(void*));
-        check(gdb_memcpy_h2d_async(dStatusPtrs_, host + 4 * n, n * sizeof(void*), stream_), "status pointers");
-        statusPtrCache_ = ptrs;
-    }
-    check(gdb_gather_words(static_cast<const uint64_t* const*>(dStatusPtrs_), static_cast<int>(n), 4,
-                           static_cast<uint64_t*>(dStatusOut_), stream_),
-          "gather status words");
-    check(gdb_memcpy_d2h_async(host, dStatusOut_, n * 32, stream_), "read status words");
+    uint64_t* host = ensurePinned(32 * pieces.size());
+    for (size_t i = 0; i < pieces.size(); i += GDB_GATHER_MAX)
+        check(gdb_gather_to_host(pieces.data() + i, static_cast<int>(std::min<size_t>(GDB_GATHER_MAX, pieces.size() - i)),
+                                 host, stream_),
+              "read status words");
     ps.host = host;
     return ps;
 }
@@ -583,7 +596,7 @@ std::vector<std::array<uint64_t, 4>> HipGenericExecutor::judgeStatuses(const Pen
 std::vector<std::array<uint64_t, 4>> HipGenericExecutor::checkStatus(const HipCodegen& cg, int firstPhase,
                                                                      int lastPhase) {
     const PendingStatus ps = enqueueStatus(cg, firstPhase, lastPhase);
-    if (!ps.refs.empty()) check(gdb_stream_sync(stream_), "gdb_stream_sync");
+    if (!ps.refs.empty()) syncStream();
     return judgeStatuses(ps);
 }
 
@@ -642,7 +655,7 @@ bool HipGenericExecutor::collectGroups(const HipResultSchema& schema, GenericRes
         if (!out) return false;
         uint64_t* w = static_cast<uint64_t*>(out.get());
         check(gdb_group_rows_small(table, slots, w, stream_), "gdb_group_rows_small");
-        check(gdb_stream_sync(stream_), "gdb_stream_sync");
+        syncStream();
         const size_t n = static_cast<size_t>(w[0]);
         if (n <= GDB_GROUP_ROWS_SMALL) {
             const uint64_t* col = w + 8;
@@ -665,7 +678,7 @@ bool HipGenericExecutor::collectGroups(const HipResultSchema& schema, GenericRes
     uint64_t* host = ensurePinned(16);
     check(gdb_group_rows_compact(table, slots, pairs, head, stream_), "gdb_group_rows_compact");
     check(gdb_memcpy_d2h_async(host, head, 16, stream_), "read group count");
-    check(gdb_stream_sync(stream_), "gdb_stream_sync");
+    syncStream();
     const uint64_t n = host[0], maxKey = host[1];
     if (n == 0) return true;
     const size_t col8 = up(static_cast<size_t>(n) * 8), col4 = up(static_cast<size_t>(n) * 4);
@@ -680,7 +693,7 @@ bool HipGenericExecutor::collectGroups(const HipResultSchema& schema, GenericRes
                               reinterpret_cast<int64_t*>(cols + at[3]), reinterpret_cast<int64_t*>(cols + at[4]), stream_),
           "gdb_group_rows_sort");
     check(gdb_memcpy_d2h_async(out.get(), cols, colBytes, stream_), "read group columns");
-    check(gdb_stream_sync(stream_), "gdb_stream_sync");
+    syncStream();
     for (size_t k = 0; k < 5; ++k) {
         auto& c = res.columns[k];
         c.hold = out;
@@ -698,11 +711,59 @@ GenericResult HipGenericExecutor::collectResult(const HipCodegen& cg) {
         GenericResult res;
         if (collectGroups(cg.getResultSchema(), res)) return res;
     }
-    check(gdb_stream_sync(stream_), "gdb_stream_sync");
+    // The few words of a small result are written to pinned memory by one
+    // launch and one wait serves them all; the collector's reads are answered
+    // from there, or by a copy when they go beyond (more rows than the piece).
+    struct Piece {
+        std::string name;
+        size_t bytes = 0, at = 0;
+    };
+    std::vector<Piece> have;
+    size_t total = 0;
+    for (const auto& b : resultBuffers(cg.getResultSchema())) {
+        auto it = buffers_.find(b.first);
+        if (it == buffers_.end()) continue;
+        const size_t bytes = std::min({b.second, it->second.bytes, size_t{16384}}) / 4 * 4;
+        if (bytes == 0) continue;
+        have.push_back({b.first, bytes, total});
+        total += (bytes + 15) / 16 * 16;
+    }
+    const char* host = nullptr;
+    if (!have.empty()) {
+        host = reinterpret_cast<const char*>(ensurePinned(total));
+        std::vector<gdb_gather_piece> pieces;
+        for (const auto& h : have)
+            pieces.push_back({buffers_.at(h.name).ptr, static_cast<uint32_t>(h.bytes), static_cast<uint32_t>(h.at)});
+        check(gdb_gather_to_host(pieces.data(), static_cast<int>(pieces.size()), ensurePinned(total), stream_),
+              "read result");
+    }
+    syncStream();
     return HipResultCollector::collect(
         cg.getResultSchema(),
-        [this](const std::string& name, size_t off, void* dst, size_t bytes) { readBuffer(name, off, dst, bytes); },
+        [&](const std::string& name, size_t off, void* dst, size_t bytes) {
+            for (const auto& h : have)
+                if (h.name == name && off + bytes <= h.bytes) {
+                    std::memcpy(dst, host + h.at + off, bytes);
+                    return;
+                }
+            readBuffer(name, off, dst, bytes);
+        },
         [this](const std::string& expr) { return sizes_.resolve(expr); });
+}
+
+std::vector<std::pair<std::string, size_t>> HipGenericExecutor::resultBuffers(const HipResultSchema& rs) const {
+    switch (rs.kind) {
+        case HipResultSchema::KEYED_AGG:
+            return {{rs.keyed.bufferName, static_cast<size_t>(rs.keyed.numBuckets) * static_cast<size_t>(rs.keyed.wordsPerBucket) * 8}};
+        case HipResultSchema::TOPK:
+            return {{rs.topk.ctlBuffer, 32}, {rs.topk.bufferName, 16 * static_cast<size_t>(rs.topk.k)}};
+        case HipResultSchema::HISTOGRAM:
+        case HipResultSchema::COUNTS:
+            return {{rs.counts.bufferName, static_cast<size_t>(sizes_.resolve(rs.counts.sizeExpr)) * 4}};
+        case HipResultSchema::ROWS:
+            return {{rs.rows.ctlBuffer, 32}, {rs.rows.bufferName, rs.rows.fields.size() * 8 * 64}};  // the first 64 rows
+        default: return {};
+    }
 }
 
 void HipGenericExecutor::releaseAllocatedBuffers() {

@@ -184,15 +184,13 @@ private:
         size_t offset = 0, bytes = 0;
     };
     std::unordered_map<std::string, Hook> hooks_;
-    // pinned host staging (hook reads, status words) and the device side of
-    // the bulk status read: the status buffers' addresses and the gathered words
+    // pinned host staging: hook reads, status words, small results
     uint64_t* pinned_ = nullptr;
     size_t pinnedBytes_ = 0;
-    void* dStatusPtrs_ = nullptr;
-    void* dStatusOut_ = nullptr;
-    size_t statusCap_ = 0;
-    std::vector<const void*> statusPtrCache_;
+    bool pinnedInFlight_ = false;  // writes to it may be enqueued and not waited for
     uint64_t* ensurePinned(size_t bytes);
+    void dropPinned();
+    void syncStream();
     std::map<std::pair<gdb_kernel, int>, int> occupancy_;
     // Hash-aggregate results (collectGroups): device workspaces, grown as
     // needed and freed with the runner's buffers, and the pinned block the
@@ -218,12 +216,15 @@ private:
     gdb_event evA_ = nullptr;
     std::vector<gdb_event> events_;
     std::vector<float> measuredPhase_, measuredFill_;
+    std::vector<bool> ownStart_;  // phases with a start event of their own (the others begin at the end before)
 
     Buffer& ensureBuffer(const HipParamBinding& b);
     void resolveBufferTables();
     void launchPhase(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq, const HipCodegen::PhaseInfo& p,
                      std::unordered_map<std::string, bool>& initDone, const std::unordered_map<std::string, const HipParamBinding*>& initSpec,
-                     unsigned* gridOut, gdb_event beforeKernel = nullptr);
+                     unsigned* gridOut, gdb_event beforeKernel, bool* marked);
+    // Buffers (and bytes) a small result of this schema reads.
+    std::vector<std::pair<std::string, size_t>> resultBuffers(const HipResultSchema& rs) const;
     std::unordered_map<std::string, const HipParamBinding*> initSpecs(const HipCodegen& cg) const;
     // Initialise, in one launch, every buffer defined by phases [first, last)
     // whose size is known now; marks them done.

@@ -271,6 +271,11 @@ struct gdb_graph_s {
     hipGraphExec_t exec = nullptr;
 };
 
+namespace {
+std::mutex g_blockMu;
+std::vector<void*> g_blocks;  // pinned blocks not in use (gdb_host_take_block)
+}  // namespace
+
 extern "C" {
 
 const char* gdb_last_error(void) { return g_err.c_str(); }
@@ -315,6 +320,11 @@ gdb_status gdb_shutdown(gdb_ctx ctx) {
     if (!ctx) return GDB_OK;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    {
+        std::lock_guard<std::mutex> lk(g_blockMu);
+        for (void* b : g_blocks) (void)hipHostFree(b);
+        g_blocks.clear();
+    }
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return GDB_OK;
@@ -375,6 +385,31 @@ gdb_status gdb_host_free_pinned(void* hptr) {
     if (!hptr) return GDB_OK;
     GDB_HIP_TRY(hipHostFree(hptr), "hipHostFree");
     return GDB_OK;
+}
+
+gdb_status gdb_host_take_block(void** hptr) {
+    if (!hptr) return fail(GDB_ERR_INVALID, "gdb_host_take_block: null output");
+    {
+        std::lock_guard<std::mutex> lk(g_blockMu);
+        if (!g_blocks.empty()) {
+            *hptr = g_blocks.back();
+            g_blocks.pop_back();
+            return GDB_OK;
+        }
+    }
+    return gdb_host_alloc_pinned(GDB_PINNED_BLOCK, hptr);
+}
+
+gdb_status gdb_host_give_block(void* hptr) {
+    if (!hptr) return GDB_OK;
+    {
+        std::lock_guard<std::mutex> lk(g_blockMu);
+        if (g_blocks.size() < GDB_PINNED_POOL) {
+            g_blocks.push_back(hptr);
+            return GDB_OK;
+        }
+    }
+    return gdb_host_free_pinned(hptr);
 }
 
 gdb_status gdb_memcpy_h2d_async(void* dst, const void* src, size_t bytes, gdb_stream s) {

@@ -83,6 +83,14 @@ gdb_status gdb_mem_info(gdb_ctx ctx, size_t* free_bytes, size_t* total_bytes);
  * zero-copy columns (src/infra.h:894-897). */
 gdb_status gdb_host_alloc_pinned(size_t bytes, void** hptr);
 gdb_status gdb_host_free_pinned(void* hptr);
+/* A pinned block of GDB_PINNED_BLOCK bytes from a process-wide pool (page-
+ * locking one takes about 40 us, more than a small query's kernels). give
+ * returns a block nothing writes any more; up to GDB_PINNED_POOL blocks are
+ * kept, and gdb_shutdown frees the ones that are not in use. */
+#define GDB_PINNED_BLOCK 32768
+#define GDB_PINNED_POOL 64
+gdb_status gdb_host_take_block(void** hptr);
+gdb_status gdb_host_give_block(void* hptr);
 
 /* Copies. Replace host memcpy/contents() access on shared buffers
  * (src/infra.h:1039; codegen/execution/metal_result_collector.cpp:170-171). */

@@ -63,6 +63,18 @@ gdb_status gdb_gen_device_uniform_i64(int64_t* out, uint64_t n, int64_t lo, int6
  * the reference (its runner reads status per query from shared memory). */
 gdb_status gdb_gather_words(const uint64_t* const* src, int n, int words, uint64_t* dst, gdb_stream st);
 
+/* Up to GDB_GATHER_MAX pieces of device memory written to pinned host memory
+ * by one small launch (pinned_dst + host_offset each, 4-byte multiples): a
+ * run's status words, or the few words of a result, with one wait and no copy
+ * engine. Read after the stream is waited for. */
+#define GDB_GATHER_MAX 48
+typedef struct gdb_gather_piece {
+    const void* src;
+    uint32_t bytes;
+    uint32_t host_offset;
+} gdb_gather_piece;
+gdb_status gdb_gather_to_host(const gdb_gather_piece* pieces, int n, void* pinned_dst, gdb_stream st);
+
 /* Groups of a hash-aggregate table in key order, as columns: slots of 4 words
  * [key | count << 32, sum, min, max], empty key 0xFFFFFFFF (the result the
  * reference's collector assembles on the host,
