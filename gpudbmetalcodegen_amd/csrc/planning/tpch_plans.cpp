@@ -57,8 +57,13 @@ HipQueryPlan tpchQ6(const PlanOptions& o) {
     auto agg = std::make_unique<HipKeyedAgg>(std::move(sel), "d_q6_sum", "0", 1);
     agg->addAggregate("revenue", AggKind::SumI64, "l_extendedprice * l_discount", 4);
     agg->addAggregate("count", AggKind::Count, "1", 0);
-    auto& ph = appendPhase(plan, "Q6_reduce", std::move(agg), optInt(o, "block", 256), optInt(o, "items", 2), {2, 4});
-    ph.launchBound = 256;
+    // Every block adds its sums to the same two result words, one after the
+    // other, so the grid's last blocks wait in line: large blocks, few of
+    // them. Blocks of 256 / 512 / 1024 at SF 1: 44-48 / 33-35 / 30-32 us, at
+    // SF 0.2 32 / 21 / 15, at SF 0.02 8.1 / 7.2 / 7.2.
+    const int block = optInt(o, "block", 1024);
+    auto& ph = appendPhase(plan, "Q6_reduce", std::move(agg), block, optInt(o, "items", 2), {2, 4});
+    ph.launchBound = std::max(256, block);
     ph.scalarParams = {"q6_date_lo", "q6_date_hi", "q6_disc_lo", "q6_disc_hi", "q6_qty_hi"};
     plan.requiredScalars = ph.scalarParams;
     plan.chunkable = true;
@@ -193,8 +198,11 @@ HipQueryPlan tpchQ12(const PlanOptions& o) {
         agg->addAggregate("high_line_count", AggKind::SumI64, "(i64)(_pcls == 2u)", 0);
         agg->addAggregate("low_line_count", AggKind::SumI64, "(i64)(_pcls != 2u)", 0);
         agg->setBucketLabels({opt(o, "mode1", "MAIL"), opt(o, "mode2", "SHIP")}, "l_shipmode");
-        auto& ph = appendPhase(plan, "Q12_count", std::move(agg), 256, 4);
-        ph.launchBound = 256;
+        // 512: half the blocks that queue at the four result words. Blocks of
+        // 256 / 512 / 1024 at SF 1: 45 / 34 / 27 us, at SF 0.2 20 / 15 / 13,
+        // at SF 0.02 7.6 / 8.0 / 9.2 (1024 leaves too few blocks there)
+        auto& ph = appendPhase(plan, "Q12_count", std::move(agg), 512, 4);
+        ph.launchBound = 512;
         ph.scalarParams = {"q12_mode1", "q12_mode2", "q12_date_lo", "q12_date_hi"};
     }
     plan.requiredScalars = {"q12_mode1", "q12_mode2", "q12_date_lo", "q12_date_hi"};
@@ -269,7 +277,10 @@ HipQueryPlan tpchQ14(const PlanOptions& o) {
         agg->addAggregate("revenue", AggKind::SumI64, kRevenue, 4);
         agg->addAggregate("count", AggKind::Count, "1", 0);
         agg->addAverage("promo_revenue", "promo_revenue_x100", "revenue");
-        auto& ph = appendPhase(plan, "Q14_sum", std::move(agg), 256, optInt(o, "items", 4));
+        // 512: half the blocks that queue at the three result words. Blocks of
+        // 256 / 512 / 1024 at SF 1: 48 / 37 / 31 us, at SF 0.2 21 / 16 / 14,
+        // at SF 0.02 7.6 / 7.4 / 8.4
+        auto& ph = appendPhase(plan, "Q14_sum", std::move(agg), 512, optInt(o, "items", 4));
         ph.scalarParams = {"q14_date_lo", "q14_date_hi"};
     }
     plan.requiredScalars = {"like_l1", "q14_date_lo", "q14_date_hi"};
