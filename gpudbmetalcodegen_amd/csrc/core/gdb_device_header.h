@@ -863,29 +863,24 @@ GDB_DEV void gdb_topk_wave_select(GdbTopK<K>& t, u64* out) {
 // Words of LDS gdb_topk_block_merge needs (blocks of up to 1024 threads).
 #define GDB_TOPK_LDS_WORDS(K) (34 * (K))
 // Block-wide top K: every wave selects its top K (no barrier), wave 0
-// selects the block's top K from the waves' lists. On return every
-// thread's list holds the block's top K, and res = lds + 32K holds it as
-// (h, l) pairs. All threads of the block must call it.
+// selects the block's top K from the waves' lists (each already sorted, so
+// lane w takes wave w's list as it stands, without an insertion). On return
+// lds + 32K holds it as (h, l) pairs. All threads of the block must call it.
 template <int K>
 GDB_DEV void gdb_topk_block_merge(GdbTopK<K>& t, u64* lds) {
     const int nw = (int)(blockDim.x >> 6);
-    u64* res = lds + 32 * K;
     gdb_topk_wave_select<K>(t, lds + 2 * K * gdb_wave());
     __syncthreads();
     if (gdb_wave() == 0) {
+        const bool own = gdb_lane() < nw;
+        const u64* list = lds + 2 * K * (own ? gdb_lane() : 0);
         GdbTopK<K> m;
-        gdb_topk_init<K>(m);
-        for (int e = gdb_lane(); e < nw * K; e += 64) {
-            const u64 h = lds[2 * e], l = lds[2 * e + 1];
-            if ((h | l) != 0) gdb_topk_push<K>(m, h, l);
-        }
-        gdb_topk_wave_select<K>(m, res);
-    }
-    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-        t.h[j] = res[2 * j];
-        t.l[j] = res[2 * j + 1];
+        for (int j = 0; j < K; ++j) {
+            m.h[j] = own ? list[2 * j] : 0ull;
+            m.l[j] = own ? list[2 * j + 1] : 0ull;
+        }
+        gdb_topk_wave_select<K>(m, lds + 32 * K);
     }
     __syncthreads();
 }

@@ -2459,7 +2459,7 @@ void HipTopKMerge::produceImpl(HipCodegen& cg, ConsumerFn consume) {
     const std::string K = s(k_);
     const std::string ctl = out_ + "_ctl";
     const std::string cand = out_ + "_cand";
-    const std::string NC = s(static_cast<long long>(k_) * HipTopK::kMaxBlocks);
+    const std::string NB = s(static_cast<long long>(HipTopK::kMaxBlocks));
     cg.setPhaseRowsExpr("1");
     cg.setPhaseMaxThreadgroups(1);
     cg.addBufferParam(out_, "u64", 8, s(2LL * k_), InitKind::Zero, {}, false, true);
@@ -2470,26 +2470,28 @@ void HipTopKMerge::produceImpl(HipCodegen& cg, ConsumerFn consume) {
         cg.declareLds("u64", "_tk_lds", "GDB_TOPK_LDS_WORDS(" + K + ")");
         cg.addLine("GdbTopK<" + K + "> _f;");
         cg.addLine("gdb_topk_init<" + K + ">(_f);");
-        // Candidates in batches of 8 per thread: the batch's 16-byte loads
-        // are all issued before the first insertion, so the (cross-XCD,
-        // uncached) candidate reads cost one round trip per batch instead of
-        // one per candidate.
-        cg.addBlock("for (u64 _c0 = 0; _c0 < " + NC + "; _c0 += 8ull * blockDim.x)", [&]() {
-            cg.addLine("u64x2 _cv[8];");
+        // A block's candidates are sorted, so a thread takes one block's list
+        // as it stands: its loads are all in flight at once and nothing is
+        // inserted (blocks of fewer threads than lists push the rest). Lists
+        // shorter than K, and those of blocks not launched, end in zeros.
+        cg.addBlock("if (threadIdx.x < " + NB + "u)", [&]() {
+            cg.addLine("const u64x2* _cl = reinterpret_cast<const u64x2*>(" + cand + ") + (u64)threadIdx.x * " + K + "ull;");
             cg.addLine("#pragma unroll");
-            cg.addLine("for (int _j = 0; _j < 8; ++_j) { const u64 _c = _c0 + (u64)_j * blockDim.x + threadIdx.x; _cv[_j] = _c < " +
-                       NC + " ? reinterpret_cast<const u64x2*>(" + cand + ")[_c] : u64x2{0ull, 0ull}; }");
-            cg.addLine("#pragma unroll");
-            cg.addLine("for (int _j = 0; _j < 8; ++_j) if ((_cv[_j].x | _cv[_j].y) != 0) gdb_topk_push<" + K +
-                       ">(_f, _cv[_j].x, _cv[_j].y);");
+            cg.addLine("for (int _j = 0; _j < " + K + "; ++_j) { const u64x2 _cv = _cl[_j]; _f.h[_j] = _cv.x; _f.l[_j] = _cv.y; }");
+        });
+        cg.addBlock("for (u32 _b = threadIdx.x + blockDim.x; _b < " + NB + "u; _b += blockDim.x)", [&]() {
+            cg.addLine("const u64x2* _cl = reinterpret_cast<const u64x2*>(" + cand + ") + (u64)_b * " + K + "ull;");
+            cg.addLine("for (int _j = 0; _j < " + K + "; ++_j) { const u64x2 _cv = _cl[_j]; if ((_cv.x | _cv.y) == 0) break; "
+                       "gdb_topk_push<" + K + ">(_f, _cv.x, _cv.y); }");
         });
         cg.addLine("gdb_topk_block_merge<" + K + ">(_f, _tk_lds);");
         cg.addLine("const u64* _tk_res = _tk_lds + 32 * " + K + ";");
-        cg.addBlock("if (threadIdx.x == 0)", [&]() {
+        cg.addBlock("if (threadIdx.x < 64u)", [&]() {
+            cg.addLine("for (u32 _j = threadIdx.x; _j < " + s(2LL * k_) + "u; _j += 64u) " + out_ + "[_j] = _tk_res[_j];");
             cg.addLine("u64 _valid = 0;");
-            cg.addLine("for (int _j = 0; _j < " + K + "; ++_j) { " + out_ + "[2 * _j] = _tk_res[2 * _j]; " + out_ +
-                       "[2 * _j + 1] = _tk_res[2 * _j + 1]; if ((_tk_res[2 * _j] | _tk_res[2 * _j + 1]) != 0) ++_valid; }");
-            cg.addLine(ctl + "[3] = _valid;");
+            cg.addLine("for (u32 _j = 0; _j < " + K + "u; _j += 64u) { const u32 _r = _j + threadIdx.x; _valid += "
+                       "(u64)__builtin_popcountll(__ballot(_r < " + K + "u && (_tk_res[2 * _r] | _tk_res[2 * _r + 1]) != 0)); }");
+            cg.addLine("if (threadIdx.x == 0) " + ctl + "[3] = _valid;");
         });
     });
     consume();

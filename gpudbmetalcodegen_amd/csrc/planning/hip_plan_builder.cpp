@@ -185,23 +185,37 @@ HipQueryPlan buildQ3(const PlanOptions& o) {
         // block of 1024 per CU then, unless block_b / block_count say otherwise)
         const int aWords = optInt(o, "a_lds_words", 0);
         probe->setLdsCache(aWords, true);
+        const int blockB = optInt(o, "block_b", aWords > 0 ? 1024 : 512), itemsB = optInt(o, "items_b", 4);
+        // compact_b=1: the rows that pass (a tenth of B at the headline
+        // filters) are queued per wave, so the insert's CAS and the bitmap's
+        // OR run lanes-dense: the round trips a wave waits for fall to one or
+        // two. B of 150K / 1.5M / 15M rows: 19.4 -> 14.8, 29.2 -> 26.2, 162 ->
+        // 162 us (there the table's lines bind it). The default where the
+        // queues take at most 32 KB of LDS and no other form is asked for.
+        const bool plainB = aWords == 0 && optInt(o, "staged", 0) == 0 && optInt(o, "prefetch", 0) == 0 &&
+                            blockB * itemsB <= 4096;
+        const bool compactB = optInt(o, "compact_b", plainB ? 1 : 0) != 0;
+        std::unique_ptr<HipOperator> rows = std::move(probe);
+        if (compactB)
+            rows = std::make_unique<HipWaveCompact>(
+                std::move(rows), std::vector<HipWaveCompact::Var>{{"i32", "b_key"}, {"i32", "b_date"}});
         std::unique_ptr<HipOperator> top =
-            std::make_unique<HipHashBuild>(std::move(probe), "d_q3_b_ht", "b_key", "b_date", "b_slots", 2);
+            std::make_unique<HipHashBuild>(std::move(rows), "d_q3_b_ht", "b_key", "b_date", "b_slots", 2);
         // bflags=1: the B-key bitmap is built as byte flags (plain stores, no
         // atomic ORs) and packed into the bitmap by the next phase
         if (probeBitmap && bflags)
             top = std::make_unique<HipByteFlagBuild>(std::move(top), "d_q3_b_flags", "b_key", "b_bits");
         else if (probeBitmap)
             top = std::make_unique<HipBitmapBuild>(std::move(top), "d_q3_b_bitmap", "b_key", "b_bits");
-        // block 512: measured 0.163 vs 0.166 ms at 256 (1024: 0.164, 128: 0.188)
-        auto& ph = appendPhase(plan, "Q3_build_b_table", std::move(top), optInt(o, "block_b", aWords > 0 ? 1024 : 512),
-                               optInt(o, "items_b", 4));
+        // block 512: measured 0.162 vs 0.166 ms at 256, 15M rows; 1.5M rows
+        // 28 vs 34 us
+        auto& ph = appendPhase(plan, "Q3_build_b_table", std::move(top), blockB, itemsB);
         ph.scalarParams = {"q3_date"};
         // staged=1 puts the home-slot CAS of a thread's ITEMS rows in flight
-        // together; per-row emission measures faster here (0.166 vs 0.177 ms
-        // at 15M rows: ~10% of the rows reach the CAS, so a batch rarely
-        // holds more than one)
-        ph.staged = optInt(o, "staged", 0) != 0;
+        // together (without the queue): 0.177 ms at 15M rows, where ~10% of
+        // the rows reach the CAS and a batch rarely holds more than one
+        ph.staged = compactB || optInt(o, "staged", 0) != 0;
+        if (compactB) ph.launchBound = blockB;  // sizes the per-wave queues
         ph.prefetch = optInt(o, "prefetch", 0) != 0;
     }
     if (probeBitmap && bflags) {
@@ -261,13 +275,17 @@ HipQueryPlan buildQ3(const PlanOptions& o) {
         top->addColumn("b_date", 1, 32, 32, 0x7FFFFFFFll);
         auto merge = top->makeMerge();
         // ITEMS slots per thread in flight (the grid is capped by the
-        // candidate lists, so per-thread depth carries the bandwidth)
-        auto& ph = appendPhase(plan, "Q3_topk", std::move(top), 256, optInt(o, "items_topk", 16), {4, 8, 16});
+        // candidate lists, so per-thread depth carries the bandwidth); 4, not
+        // 16: a small table then takes more blocks and fewer serial
+        // insertions a thread (32K slots: 16 / 8 / 4 give 16.4 / 13.5 / 11.8 us,
+        // 4M slots 33.5 / 33.5 / 32.9)
+        auto& ph = appendPhase(plan, "Q3_topk", std::move(top), 256, optInt(o, "items_topk", 4), {4, 8, 16});
         ph.launchBound = 256;
-        // one block merges every candidate list: 1024 threads keep each
-        // thread's serial insertion chain short
-        auto& pm = appendPhase(plan, "Q3_topk_merge", std::move(merge), optInt(o, "merge_block", 1024), 1, {1});
-        pm.launchBound = 1024;
+        // one block merges every candidate list, one list a thread (1024
+        // threads, inserting candidates one by one: 16-19 us; now 11-12)
+        const int mergeBlock = optInt(o, "merge_block", HipTopK::kMaxBlocks);
+        auto& pm = appendPhase(plan, "Q3_topk_merge", std::move(merge), mergeBlock, 1, {1});
+        pm.launchBound = std::max<int>(HipTopK::kMaxBlocks, mergeBlock);
     }
     plan.requiredScalars = {"q3_seg", "q3_date"};
     plan.requiredSymbols = {"a_bits", "b_bits"};

@@ -115,13 +115,17 @@ HipQueryPlan tpchQ3(const PlanOptions& o) {
         top->addColumn("o_orderdate", 1, 32, 32, 0x7FFFFFFFll, 0, true);
         auto merge = top->makeMerge();
         // ITEMS slots per thread in flight (the grid is capped by the
-        // candidate lists, so per-thread depth carries the bandwidth)
-        auto& ph = appendPhase(plan, "Q3_topk", std::move(top), 256, optInt(o, "items_topk", 16), {4, 8, 16});
+        // candidate lists, so per-thread depth carries the bandwidth); 4, not
+        // 16: a small table then takes more blocks and fewer serial
+        // insertions a thread (32K slots: 16 / 8 / 4 give 16.4 / 13.5 / 11.8 us,
+        // 4M slots 33.5 / 33.5 / 32.9)
+        auto& ph = appendPhase(plan, "Q3_topk", std::move(top), 256, optInt(o, "items_topk", 4), {4, 8, 16});
         ph.launchBound = 256;
-        // one block merges every candidate list: 1024 threads keep each
-        // thread's serial insertion chain short
-        auto& pm = appendPhase(plan, "Q3_topk_merge", std::move(merge), optInt(o, "merge_block", 1024), 1, {1});
-        pm.launchBound = 1024;
+        // one block merges every candidate list, one list a thread (1024
+        // threads, inserting candidates one by one: 16-19 us; now 11-12)
+        const int mergeBlock = optInt(o, "merge_block", HipTopK::kMaxBlocks);
+        auto& pm = appendPhase(plan, "Q3_topk_merge", std::move(merge), mergeBlock, 1, {1});
+        pm.launchBound = std::max<int>(HipTopK::kMaxBlocks, mergeBlock);
     }
     plan.requiredScalars = {"q3_seg", "q3_date"};
     plan.requiredSymbols = {"c_bits", "o_bits", "o_slots"};
@@ -487,9 +491,9 @@ HipQueryPlan tpchQ10(const PlanOptions& o) {
         auto merge = top->makeMerge();
         auto& ph = appendPhase(plan, "Q10_topk", std::move(top), 256, 4);
         ph.launchBound = 256;
-        // K = 20 lists need more than the 128 VGPRs a 1024-thread block allows
-        auto& pm = appendPhase(plan, "Q10_topk_merge", std::move(merge), 256, 1, {1});
-        pm.launchBound = 256;
+        // one candidate list a thread (K = 20 lists fit the 256 VGPRs of a 512-thread block)
+        auto& pm = appendPhase(plan, "Q10_topk_merge", std::move(merge), HipTopK::kMaxBlocks, 1, {1});
+        pm.launchBound = HipTopK::kMaxBlocks;
     }
     plan.requiredScalars = {"q10_date_lo", "q10_date_hi", "q10_flag"};
     plan.requiredSymbols = {"o_bits", "c_bits"};
