@@ -183,6 +183,7 @@ def load() -> tuple[C.CDLL, C.CDLL]:
     _sig(eng, "gdb_executor_owned_bytes", [vp, P(sz)])
     _sig(eng, "gdb_executor_release", [vp])
     _sig(eng, "gdb_executor_collect", [vp, vp, P(vp)])
+    _sig(eng, "gdb_executor_collect_many", [P(vp), P(vp), C.c_int, P(vp)])
     _sig(eng, "gdb_result_shape", [vp, P(u64), P(i32)])
     _sig(eng, "gdb_result_column", [vp, i32, vp, sz, P(i32)])
     _sig(eng, "gdb_result_i64", [vp, i32, vp])

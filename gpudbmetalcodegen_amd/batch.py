@@ -248,11 +248,9 @@ class Workload3:
         return (time.perf_counter() - t0) * 1e3
 
     def results(self) -> list[dict]:
-        out = []
-        for i, s in enumerate(self.specs):
-            res = self.execs[i].collect(self.plans[s.kind], canonical=False)
-            out.append({k: np.asarray(v) for k, v in res.columns.items()})
-        return out
+        runs = [(self.execs[i], self.plans[s.kind]) for i, s in enumerate(self.specs)]
+        return [{k: np.asarray(v) for k, v in res.columns.items()}
+                for res in E.HipGenericExecutor.collect_many(runs, canonical=False)]
 
     # --- batched form ----------------------------------------------------
     def build_batch(self, block: int, chunk_rows: int = 32768, grid: int = 0, fold_rows: int = 0) -> "Batch":

@@ -606,6 +606,21 @@ gdb_status gdb_executor_collect(gdb_executor ex, gdb_plan p, gdb_result* out) {
     });
 }
 
+gdb_status gdb_executor_collect_many(const gdb_executor* ex, const gdb_plan* p, int n, gdb_result* out) {
+    return guard([&]() -> gdb_status {
+        std::vector<std::pair<HipGenericExecutor*, const HipCodegen*>> runs;
+        for (int i = 0; i < n; ++i) runs.push_back({ex[i]->ex.get(), &p[i]->cg});
+        auto results = HipGenericExecutor::collectMany(runs);
+        std::vector<std::unique_ptr<gdb_result_s>> made;
+        for (auto& r : results) {
+            made.push_back(std::make_unique<gdb_result_s>());
+            made.back()->r = std::move(r);
+        }
+        for (int i = 0; i < n; ++i) out[i] = made[static_cast<size_t>(i)].release();
+        return GDB_OK;
+    });
+}
+
 gdb_status gdb_result_shape(gdb_result r, uint64_t* rows, int* cols) {
     if (rows) *rows = r->r.rows();
     if (cols) *cols = static_cast<int>(r->r.columns.size());

@@ -629,6 +629,40 @@ std::shared_ptr<void> HipGenericExecutor::stagingFor(size_t bytes) {
     return p;
 }
 
+namespace {
+void groupColumns(const HipResultSchema& schema, GenericResult& res) {
+    static const char* const names[4] = {"count", "sum", "min", "max"};
+    res.columns.assign(5, ResultColumn{});
+    res.columns[0].name = schema.hash.keyName;
+    for (size_t k = 0; k < 4; ++k) res.columns[k + 1].name = names[k];
+}
+}  // namespace
+
+const uint64_t* HipGenericExecutor::groupTable(const HipResultSchema& schema, uint64_t* slots) const {
+    const auto& h = schema.hash;
+    const auto it = buffers_.find(h.tableName);
+    if (h.slotWords != 4 || it == buffers_.end()) return nullptr;
+    *slots = sizes_.resolve(h.slotsSymbol);
+    if (*slots > kMaxGroupSlots || *slots * 32 > it->second.bytes) return nullptr;
+    return static_cast<const uint64_t*>(it->second.ptr);
+}
+
+// The columns of what gdb_group_rows_small wrote; false when it was too much.
+bool HipGenericExecutor::smallGroups(const HipResultSchema& schema, const uint64_t* w, GenericResult& res) {
+    const size_t n = static_cast<size_t>(w[0]);
+    if (n > GDB_GROUP_ROWS_SMALL) return false;
+    groupColumns(schema, res);
+    const uint64_t* col = w + 8;
+    for (auto& c : res.columns) c.i64.resize(n);
+    for (size_t r = 0; r < n; ++r) {
+        res.columns[0].i64[r] = static_cast<int64_t>(col[r] & 0xFFFFFFFFull);
+        res.columns[1].i64[r] = static_cast<int64_t>(col[r] >> 32);
+    }
+    for (size_t k = 1; k < 4; ++k)
+        if (n) std::memcpy(res.columns[k + 1].i64.data(), col + k * GDB_GROUP_ROWS_SMALL, n * 8);
+    return true;
+}
+
 // The groups of a hash-aggregate table, ordered and split into columns on the
 // device, so only the result crosses the link (32 bytes a group instead of 32
 // a slot, from pinned memory) and the host sorts nothing. A group-by of 40M
@@ -639,36 +673,18 @@ std::shared_ptr<void> HipGenericExecutor::stagingFor(size_t bytes) {
 // that block busy longer than the general path's dozen launches take. False
 // when the workspace cannot be had (the caller reads the table instead).
 bool HipGenericExecutor::collectGroups(const HipResultSchema& schema, GenericResult& res) {
-    const auto& h = schema.hash;
-    const auto it = buffers_.find(h.tableName);
-    if (h.slotWords != 4 || it == buffers_.end()) return false;
-    const uint64_t slots = sizes_.resolve(h.slotsSymbol);
-    if (slots > kMaxGroupSlots || slots * 32 > it->second.bytes) return false;
-    const uint64_t* table = static_cast<const uint64_t*>(it->second.ptr);
-    static const char* const names[4] = {"count", "sum", "min", "max"};
-    res.columns.assign(5, ResultColumn{});
-    res.columns[0].name = h.keyName;
-    for (size_t k = 0; k < 4; ++k) res.columns[k + 1].name = names[k];
-
+    uint64_t slots = 0;
+    const uint64_t* table = groupTable(schema, &slots);
+    if (!table) return false;
     if (slots <= 2 * GDB_GROUP_ROWS_SMALL) {
         auto out = stagingFor(GDB_GROUP_ROWS_SMALL_BYTES);
         if (!out) return false;
         uint64_t* w = static_cast<uint64_t*>(out.get());
         check(gdb_group_rows_small(table, slots, w, stream_), "gdb_group_rows_small");
         syncStream();
-        const size_t n = static_cast<size_t>(w[0]);
-        if (n <= GDB_GROUP_ROWS_SMALL) {
-            const uint64_t* col = w + 8;
-            for (auto& c : res.columns) c.i64.resize(n);
-            for (size_t r = 0; r < n; ++r) {
-                res.columns[0].i64[r] = static_cast<int64_t>(col[r] & 0xFFFFFFFFull);
-                res.columns[1].i64[r] = static_cast<int64_t>(col[r] >> 32);
-            }
-            for (size_t k = 1; k < 4; ++k)
-                std::memcpy(res.columns[k + 1].i64.data(), col + k * GDB_GROUP_ROWS_SMALL, n * 8);
-            return true;
-        }
+        if (smallGroups(schema, w, res)) return true;
     }
+    groupColumns(schema, res);
 
     // workspaces: head | pairs; once the number of groups is known, sort scratch | columns
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -714,32 +730,39 @@ GenericResult HipGenericExecutor::collectResult(const HipCodegen& cg) {
     // The few words of a small result are written to pinned memory by one
     // launch and one wait serves them all; the collector's reads are answered
     // from there, or by a copy when they go beyond (more rows than the piece).
-    struct Piece {
-        std::string name;
-        size_t bytes = 0, at = 0;
-    };
-    std::vector<Piece> have;
     size_t total = 0;
-    for (const auto& b : resultBuffers(cg.getResultSchema())) {
+    const auto have = resultPieces(cg.getResultSchema(), &total);
+    const char* host = nullptr;
+    if (!have.empty()) {
+        uint64_t* pinned = ensurePinned(total);
+        host = reinterpret_cast<const char*>(pinned);
+        std::vector<gdb_gather_piece> pieces;
+        for (const auto& h : have)
+            pieces.push_back({buffers_.at(h.name).ptr, static_cast<uint32_t>(h.bytes), static_cast<uint32_t>(h.at)});
+        check(gdb_gather_to_host(pieces.data(), static_cast<int>(pieces.size()), pinned, stream_), "read result");
+    }
+    syncStream();
+    return collectPieces(cg.getResultSchema(), have, host);
+}
+
+std::vector<HipGenericExecutor::Piece> HipGenericExecutor::resultPieces(const HipResultSchema& schema,
+                                                                        size_t* total) const {
+    std::vector<Piece> have;
+    for (const auto& b : resultBuffers(schema)) {
         auto it = buffers_.find(b.first);
         if (it == buffers_.end()) continue;
         const size_t bytes = std::min({b.second, it->second.bytes, size_t{16384}}) / 4 * 4;
         if (bytes == 0) continue;
-        have.push_back({b.first, bytes, total});
-        total += (bytes + 15) / 16 * 16;
+        have.push_back({b.first, bytes, *total});
+        *total += (bytes + 15) / 16 * 16;
     }
-    const char* host = nullptr;
-    if (!have.empty()) {
-        host = reinterpret_cast<const char*>(ensurePinned(total));
-        std::vector<gdb_gather_piece> pieces;
-        for (const auto& h : have)
-            pieces.push_back({buffers_.at(h.name).ptr, static_cast<uint32_t>(h.bytes), static_cast<uint32_t>(h.at)});
-        check(gdb_gather_to_host(pieces.data(), static_cast<int>(pieces.size()), ensurePinned(total), stream_),
-              "read result");
-    }
-    syncStream();
+    return have;
+}
+
+GenericResult HipGenericExecutor::collectPieces(const HipResultSchema& schema, const std::vector<Piece>& have,
+                                                const char* host) {
     return HipResultCollector::collect(
-        cg.getResultSchema(),
+        schema,
         [&](const std::string& name, size_t off, void* dst, size_t bytes) {
             for (const auto& h : have)
                 if (h.name == name && off + bytes <= h.bytes) {
@@ -749,6 +772,77 @@ GenericResult HipGenericExecutor::collectResult(const HipCodegen& cg) {
             readBuffer(name, off, dst, bytes);
         },
         [this](const std::string& expr) { return sizes_.resolve(expr); });
+}
+
+// A batch of 64 pipelines whose results were read one by one spent 34 us on
+// each, most of it a launch and a wait: with one launch for the 32 group
+// tables, one for the others' words and one wait, replay and results take
+// 1.09 ms instead of 2.64. A result with more than kPieces bytes to read, another
+// context or stream than the first runner's, or too many groups is collected
+// by itself afterwards (the shared pinned block is free again then).
+std::vector<GenericResult> HipGenericExecutor::collectMany(
+    const std::vector<std::pair<HipGenericExecutor*, const HipCodegen*>>& runs) {
+    constexpr size_t kPieces = 1024;
+    std::vector<GenericResult> res(runs.size());
+    if (runs.empty()) return res;
+    HipGenericExecutor& first = *runs[0].first;
+    enum Way { ALONE, GROUPS, PIECES };
+    std::vector<Way> way(runs.size(), ALONE);
+    std::vector<std::shared_ptr<void>> staged(runs.size());
+    std::vector<std::vector<Piece>> have(runs.size());
+    std::vector<gdb_group_table> tables;
+    std::vector<gdb_gather_piece> pieces;
+    size_t total = 0;
+    for (size_t i = 0; i < runs.size(); ++i) {
+        HipGenericExecutor& ex = *runs[i].first;
+        const HipResultSchema& schema = runs[i].second->getResultSchema();
+        if (ex.ctx_ != first.ctx_ || ex.stream_ != first.stream_) continue;
+        if (schema.kind == HipResultSchema::HASH_AGG) {
+            uint64_t slots = 0;
+            const uint64_t* table = ex.groupTable(schema, &slots);
+            if (!table || slots > 2 * GDB_GROUP_ROWS_SMALL) continue;
+            staged[i] = ex.stagingFor(GDB_GROUP_ROWS_SMALL_BYTES);
+            if (!staged[i]) continue;
+            tables.push_back({table, static_cast<uint64_t*>(staged[i].get()), slots});
+            way[i] = GROUPS;
+            continue;
+        }
+        size_t bytes = 0;
+        auto own = ex.resultPieces(schema, &bytes);
+        if (own.empty() || bytes > kPieces) continue;
+        for (auto& h : own) {
+            h.at += total;
+            pieces.push_back({ex.buffers_.at(h.name).ptr, static_cast<uint32_t>(h.bytes), static_cast<uint32_t>(h.at)});
+        }
+        total += bytes;
+        have[i] = std::move(own);
+        way[i] = PIECES;
+    }
+    const char* host = nullptr;
+    if (!tables.empty())
+        check(gdb_group_rows_small_many(tables.data(), static_cast<int>(tables.size()), first.stream_),
+              "gdb_group_rows_small_many");
+    if (!pieces.empty()) {
+        uint64_t* pinned = first.ensurePinned(total);
+        host = reinterpret_cast<const char*>(pinned);
+        for (size_t at = 0; at < pieces.size(); at += GDB_GATHER_MAX)
+            check(gdb_gather_to_host(pieces.data() + at,
+                                     static_cast<int>(std::min<size_t>(GDB_GATHER_MAX, pieces.size() - at)), pinned,
+                                     first.stream_),
+                  "read results");
+    }
+    if (!tables.empty() || !pieces.empty()) first.syncStream();
+    for (size_t i = 0; i < runs.size(); ++i) {
+        const HipResultSchema& schema = runs[i].second->getResultSchema();
+        if (way[i] == PIECES)
+            res[i] = runs[i].first->collectPieces(schema, have[i], host);
+        else if (way[i] == GROUPS && !smallGroups(schema, static_cast<uint64_t*>(staged[i].get()), res[i]))
+            way[i] = ALONE;
+        staged[i].reset();
+    }
+    for (size_t i = 0; i < runs.size(); ++i)
+        if (way[i] == ALONE) res[i] = runs[i].first->collectResult(*runs[i].second);
+    return res;
 }
 
 std::vector<std::pair<std::string, size_t>> HipGenericExecutor::resultBuffers(const HipResultSchema& rs) const {

@@ -145,6 +145,10 @@ public:
     std::vector<std::array<uint64_t, 4>> judgeStatuses(const PendingStatus& ps) const;
 
     GenericResult collectResult(const HipCodegen& cg);
+    // The results of several runners. Small ones on one stream share a launch
+    // of each kind and one wait; every other is collected by itself.
+    static std::vector<GenericResult> collectMany(
+        const std::vector<std::pair<HipGenericExecutor*, const HipCodegen*>>& runs);
     void releaseAllocatedBuffers();
     void* getAllocatedBuffer(const std::string& name) const;
     size_t getAllocatedBytes(const std::string& name) const;
@@ -210,6 +214,14 @@ private:
     void freeWorkspace(Workspace& w);
     std::shared_ptr<void> stagingFor(size_t bytes);
     bool collectGroups(const HipResultSchema& schema, GenericResult& res);
+    const uint64_t* groupTable(const HipResultSchema& schema, uint64_t* slots) const;  // null: the host reads the table
+    static bool smallGroups(const HipResultSchema& schema, const uint64_t* w, GenericResult& res);
+    struct Piece {  // the start of a result buffer, read to the host at `at`
+        std::string name;
+        size_t bytes = 0, at = 0;
+    };
+    std::vector<Piece> resultPieces(const HipResultSchema& schema, size_t* total) const;
+    GenericResult collectPieces(const HipResultSchema& schema, const std::vector<Piece>& have, const char* host);
     bool skipInit_ = false;
     bool phaseTiming_ = true;
     std::vector<std::string> lateSymbols_;

@@ -10,6 +10,7 @@
 #include "gdb/gdb_kernels.h"
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 
 #include <string>
 
@@ -42,8 +43,7 @@ __device__ __forceinline__ u64 lanesBelow() { return (1ull << lane()) - 1ull; }
 // Bound by latency, not bytes: at 2,048 slots and 700 groups the launch, the
 // 4 loads per thread in flight together and 55 bitonic steps. The rows go
 // straight to pinned host memory, so the caller waits once and copies nothing.
-__global__ void __launch_bounds__(1024) groupRowsSmallKernel(const u64* __restrict__ tab, u32 slots,
-                                                             u64* __restrict__ out) {
+__device__ __forceinline__ void groupRowsSmall(const u64* __restrict__ tab, u32 slots, u64* __restrict__ out) {
     __shared__ u64 e[kSmallRows];
     __shared__ u32 n_;
     if (threadIdx.x == 0) n_ = 0;
@@ -99,6 +99,18 @@ __global__ void __launch_bounds__(1024) groupRowsSmallKernel(const u64* __restri
         col[3 * kSmallRows + i] = r[3];
     }
     if (threadIdx.x == 0) out[0] = n;
+}
+__global__ void __launch_bounds__(1024) groupRowsSmallKernel(const u64* tab, u32 slots, u64* out) {
+    groupRowsSmall(tab, slots, out);
+}
+// Several tables, one block each: they share one launch and one wait, and the
+// blocks' latency chains run side by side.
+struct GroupTables {
+    gdb_group_table t[GDB_GROUP_MANY];
+};
+__global__ void __launch_bounds__(1024) groupRowsSmallManyKernel(GroupTables all) {
+    const gdb_group_table& t = all.t[blockIdx.x];
+    groupRowsSmall((const u64*)t.table, (u32)t.slots, (u64*)t.pinned_out);
 }
 
 // --- general tables ---------------------------------------------------------
@@ -299,6 +311,21 @@ gdb_status gdb_group_rows_small(const uint64_t* table, uint64_t slots, uint64_t*
     hipLaunchKernelGGL(groupRowsSmallKernel, dim3(1), dim3(1024), 0, (hipStream_t)s, (const u64*)table, (u32)slots,
                        (u64*)pinned_out);
     return launched("groupRowsSmallKernel");
+}
+
+gdb_status gdb_group_rows_small_many(const gdb_group_table* tables, int n, gdb_stream s) {
+    if (n < 0 || (n > 0 && !tables)) return bad("gdb_group_rows_small_many: null argument");
+    for (int i = 0; i < n; ++i) {
+        if (!tables[i].table || !tables[i].pinned_out) return bad("gdb_group_rows_small_many: null argument");
+        if (tables[i].slots > 2 * (uint64_t)kSmallRows) return bad("gdb_group_rows_small_many: too many slots");
+    }
+    for (int i = 0; i < n; i += GDB_GROUP_MANY) {
+        GroupTables all{};
+        const int m = std::min(n - i, GDB_GROUP_MANY);
+        std::copy(tables + i, tables + i + m, all.t);
+        hipLaunchKernelGGL(groupRowsSmallManyKernel, dim3((u32)m), dim3(1024), 0, (hipStream_t)s, all);
+    }
+    return launched("groupRowsSmallManyKernel");
 }
 
 gdb_status gdb_group_rows_compact(const uint64_t* table, uint64_t slots, uint64_t* pairs, uint64_t* head, gdb_stream s) {

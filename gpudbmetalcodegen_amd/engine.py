@@ -402,9 +402,36 @@ class HipGenericExecutor:
     def collect(self, plan: HipQueryPlan, canonical: bool = True) -> GenericResult:
         """The plan's result on the host; canonical=False leaves its CSV text
         out (for callers that only take the columns)."""
-        eng = _eng()
         r = C.c_void_p()
-        N.eng_check(eng.gdb_executor_collect(self._h, plan.handle, C.byref(r)))
+        N.eng_check(_eng().gdb_executor_collect(self._h, plan.handle, C.byref(r)))
+        return self._result(r, canonical)
+
+    @classmethod
+    def collect_many(cls, runs: list, canonical: bool = True) -> list:
+        """The results of several (runner, plan) pairs, as collect() gives
+        them; small results on one stream are read with one wait."""
+        n = len(runs)
+        if n == 0:
+            return []
+        out = (C.c_void_p * n)()
+        N.eng_check(_eng().gdb_executor_collect_many((C.c_void_p * n)(*[ex._h for ex, _ in runs]),
+                                                     (C.c_void_p * n)(*[p.handle for _, p in runs]), n, out))
+        res = []
+        try:
+            while len(res) < n:
+                k = len(res)
+                r, out[k] = C.c_void_p(out[k]), None
+                res.append(cls._result(r, canonical))
+        finally:
+            for r in out[len(res):]:
+                if r:
+                    _eng().gdb_result_free(C.c_void_p(r))
+        return res
+
+    @classmethod
+    def _result(cls, r, canonical: bool) -> GenericResult:
+        """Reads a result and frees it."""
+        eng = _eng()
         try:
             head = N.two_call_string(eng.gdb_result_describe, r, guess=4096).split("\x1e")
             rows = int(head[0])
@@ -432,7 +459,7 @@ class HipGenericExecutor:
                     w = w.tolist()
                     a = np.array([(lo & 0xFFFFFFFFFFFFFFFF) + (hi << 64) for lo, hi in zip(w[::2], w[1::2])], dtype=object)
                 else:
-                    a = np.array(c[4:] if len(c) == 4 + rows else self._strings(r, i, rows), dtype=object)
+                    a = np.array(c[4:] if len(c) == 4 + rows else cls._strings(r, i, rows), dtype=object)
                 at += n
                 out[c[0]] = a
                 fmts[c[0]] = (int(c[2]), c[3] == "1")

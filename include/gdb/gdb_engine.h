@@ -171,6 +171,10 @@ gdb_status gdb_executor_release(gdb_executor ex);
 
 /* ---- Result API (GenericResult, metal_result_collector.h:19-60) ---- */
 gdb_status gdb_executor_collect(gdb_executor ex, gdb_plan p, gdb_result* out);
+/* The results of n runners, as n calls of gdb_executor_collect give them; the
+ * small ones of one stream are read with one launch of each kind and one wait.
+ * On an error no result is returned. */
+gdb_status gdb_executor_collect_many(const gdb_executor* ex, const gdb_plan* p, int n, gdb_result* out);
 gdb_status gdb_result_shape(gdb_result r, uint64_t* rows, int* cols);
 /* type: 0 = int64, 1 = int128 (two int64 per row: low word, high word), 2 = string */
 gdb_status gdb_result_column(gdb_result r, int idx, char* name, size_t cap, int* type);

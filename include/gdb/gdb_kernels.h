@@ -94,6 +94,15 @@ gdb_status gdb_gather_to_host(const gdb_gather_piece* pieces, int n, void* pinne
 #define GDB_GROUP_ROWS_SMALL_BYTES ((8 + 4 * GDB_GROUP_ROWS_SMALL) * 8)
 const char* gdb_group_rows_last_error(void);
 gdb_status gdb_group_rows_small(const uint64_t* table, uint64_t slots, uint64_t* pinned_out, gdb_stream s);
+/* The same for any number of tables, one block each and GDB_GROUP_MANY of
+ * them a launch. */
+#define GDB_GROUP_MANY 64
+typedef struct gdb_group_table {
+    const uint64_t* table;
+    uint64_t* pinned_out;
+    uint64_t slots;
+} gdb_group_table;
+gdb_status gdb_group_rows_small_many(const gdb_group_table* tables, int n, gdb_stream s);
 gdb_status gdb_group_rows_compact(const uint64_t* table, uint64_t slots, uint64_t* pairs, uint64_t* head, gdb_stream s);
 size_t gdb_group_rows_scratch_bytes(uint64_t n);
 gdb_status gdb_group_rows_sort(const uint64_t* table, uint64_t* pairs, uint64_t n, uint64_t max_key, void* scratch,
