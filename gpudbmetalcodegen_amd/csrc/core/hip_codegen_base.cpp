@@ -85,6 +85,11 @@ void HipCodegen::setPhaseCheck(const std::string& checkBuffer, const std::string
     p.checkBuffer = checkBuffer;
     p.checkMessage = message;
 }
+void HipCodegen::setPhasePartials(const std::string& symbol, bool folds) {
+    auto& p = cur("setPhasePartials");
+    p.partialsSymbol = symbol;
+    p.foldsPartials = folds;
+}
 
 // --- parameters -------------------------------------------------------------
 

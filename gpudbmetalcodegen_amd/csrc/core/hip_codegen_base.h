@@ -95,6 +95,8 @@ public:
     // A row check's status words (HipRowCheck): the run fails with `message`
     // when any row of the phase failed it.
     void setPhaseCheck(const std::string& checkBuffer, const std::string& message);
+    // The phase leaves (or, with folds, folds) up to `symbol` partial tables.
+    void setPhasePartials(const std::string& symbol, bool folds);
 
     // --- parameters ---
     // Column of a registered table; returns the pointer parameter name.
@@ -183,6 +185,10 @@ public:
         std::string ldsBytesExpr = "0u";  // range mode: LDS bytes of the body (constant expression)
         bool staged = false;              // item-batched emission (hip_operators.h)
         bool prefetch = false;            // scans load the next tile before processing this one
+        // Set on a phase that leaves partial tables and on the later phase that
+        // folds them: the symbol parameter that holds how many there may be.
+        std::string partialsSymbol;
+        bool foldsPartials = false;
         std::vector<HipParamBinding> bindings;
     };
     const std::vector<PhaseInfo>& getPhases() const { return phases_; }

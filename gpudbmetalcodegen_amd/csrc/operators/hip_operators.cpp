@@ -1808,6 +1808,7 @@ void HipHashGroupBy::produceImpl(HipCodegen& cg, ConsumerFn consume) {
             cg.addBufferParam(PM, "u64", 8, "(" + partialsMax_ + ") * " + s(ldsSlots_ / 64), InitKind::None, {}, false, true);
             cg.addBufferParam(PN, "u64", 8, "2", InitKind::Zero, {}, false, true);
             cg.addSymbolParam(NP, partialsMax_);
+            cg.setPhasePartials(NP, false);
             cg.addComment("the LDS table becomes partial table _pi, if one is left");
             cg.declareLds("u64", "_pti_" + T, "1");
             // a launch of a few blocks merges each key a few times: the fold
@@ -1860,6 +1861,7 @@ void HipGroupByMerge::produceImpl(HipCodegen& cg, ConsumerFn consume) {
     cg.addBufferParam(PM, "u64", 8, "(" + partialsMax_ + ") * " + s(ldsSlots_ / 64), InitKind::None, {}, true, true);
     cg.addBufferParam(PN, "u64", 8, "2", InitKind::Zero, {}, false, true);
     cg.addSymbolParam(NP, partialsMax_);
+    cg.setPhasePartials(NP, true);
     cg.setPhaseRowsExpr("(" + partialsMax_ + ") * " + CAP);
     cg.addComment("GroupByMerge " + T + ": a block takes a range of home slots over every partial table, so each key "
                   "reaches the global table once");

@@ -13,6 +13,17 @@ TuneResult autotunePhase(HipGenericExecutor& ex, RuntimeCompiler& rc, const Runt
                          const std::string& scalarName, const std::vector<int64_t>& scalarValues, int trials) {
     auto& ph = cg.getPhasesMutable().at(static_cast<size_t>(phase));
     const int saveBlock = ph.threadgroupSize, saveItems = ph.items;
+    // A fold consumes the partial tables that its scan leaves, so the two run
+    // together in every trial (a fold alone would find none after the first);
+    // the time taken is the tuned phase's.
+    int first = phase, last = phase + 1;
+    const auto& phases = cg.getPhases();
+    for (int i = 0; !ph.partialsSymbol.empty() && i < static_cast<int>(phases.size()); ++i)
+        if (phases[static_cast<size_t>(i)].partialsSymbol == ph.partialsSymbol) {
+            first = std::min(first, i);
+            last = std::max(last, i + 1);
+        }
+    const size_t at = static_cast<size_t>(phase - first);
     std::vector<int64_t> svals = scalarName.empty() ? std::vector<int64_t>{0} : scalarValues;
     TuneResult best;
     best.ms = std::numeric_limits<float>::infinity();
@@ -26,11 +37,11 @@ TuneResult autotunePhase(HipGenericExecutor& ex, RuntimeCompiler& rc, const Runt
                 if (!scalarName.empty()) ex.registerScalarInt(scalarName, sv);
                 double p50 = std::numeric_limits<double>::infinity();
                 try {
-                    ex.execute(rc, cq, cg, 1, 1, phase, phase + 1);  // untimed warmup
+                    ex.execute(rc, cq, cg, 1, 1, first, last);  // untimed warmup
                     std::vector<double> t;
                     for (int k = 0; k < std::max(2, trials); ++k) {
-                        auto r = ex.execute(rc, cq, cg, 0, 1, phase, phase + 1);
-                        t.push_back(r.phaseTimesMs.empty() ? 0.0 : r.phaseTimesMs[0]);
+                        auto r = ex.execute(rc, cq, cg, 0, 1, first, last);
+                        t.push_back(r.phaseTimesMs.size() > at ? r.phaseTimesMs[at] : 0.0);
                     }
                     std::sort(t.begin(), t.end());
                     t.pop_back();  // drop the slowest

@@ -7,7 +7,8 @@
 // block size, ITEMS per thread (a compiled variant of the phase) and one
 // optional runtime scalar (e.g. the LDS hash slots in use, as log2). The
 // candidate set is the cross product; the phase's kernel time comes from
-// events around the kernel alone.
+// events around the kernel alone. Phases that leave and fold partial tables
+// run together, whichever of them is tuned.
 
 #include "../execution/hip_generic_executor.h"
 #include "../execution/runtime_compiler.h"

@@ -2,11 +2,14 @@
 sort where it can go wrong — few blocks (no partials), LDS tables smaller
 than the groups (spills, keys probing past their home slot and round the
 table's end), tables filled over several runs or chunks, and as work items of
-a batch."""
+a batch; and the fold's launch shape tuned."""
+
+import ctypes as C
 
 import numpy as np
 import pytest
 
+from gpudbmetalcodegen_amd import _native as N
 from gpudbmetalcodegen_amd import batch as B
 from gpudbmetalcodegen_amd import engine as E
 from gpudbmetalcodegen_amd import queries as Q
@@ -79,3 +82,34 @@ def test_fold_of_batched_pipelines(ctx, chunk, lds_bits):
             b.close()
     finally:
         w.close()
+
+
+def _autotune(ex, plan, phase, blocks, items):
+    bl, it = (C.c_int * len(blocks))(*blocks), (C.c_int * len(items))(*items)
+    block, n, ms, count = C.c_int(), C.c_int(), C.c_float(), C.c_int()
+    table = (C.c_double * (4 * len(blocks) * len(items)))()
+    N.eng_check(N.load()[1].gdb_autotune_phase(ex.handle, plan.handle, phase.encode(), bl, len(blocks), it, len(items),
+                                               None, None, 0, 3, C.byref(block), C.byref(n), None, C.byref(ms), table,
+                                               C.byref(count)))
+    assert block.value in blocks and ms.value > 0
+    return count.value
+
+
+@pytest.mark.parametrize("phase", ["GB_agg", "GB_merge"])
+def test_autotuned_fold_folds_in_every_trial(ctx, phase):
+    """Each trial fills and folds partials: after tuning, the group table holds
+    the rows of the table registered by then, not those of the run before."""
+    first, second = _table(300_001, 900, 1), _table(300_001, 400, 2)
+    dev = Q.upload_tables(ctx, {"G": first})
+    other = Q.upload_tables(ctx, {"G": second})
+    try:
+        run = Q.run_groupby(ctx, dev, slots=2048, variant="lds")
+        _same(run.result.columns, first)
+        shape = run.plan.get_launch(phase)
+        run.executor.register_table(other["G"])
+        assert _autotune(run.executor, run.plan, phase, (64, 256, 1024), [shape[1]]) == 3
+        _same(run.executor.collect(run.plan).columns, second)
+        run.plan.set_launch(phase, *shape)
+    finally:
+        dev["G"].free(ctx)
+        other["G"].free(ctx)
