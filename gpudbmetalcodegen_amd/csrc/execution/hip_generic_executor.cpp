@@ -267,7 +267,7 @@ void HipGenericExecutor::prepare(const HipCodegen& cg, int firstPhase, int lastP
 void HipGenericExecutor::launchPhase(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq,
                                      const HipCodegen::PhaseInfo& p, std::unordered_map<std::string, bool>& initDone,
                                      const std::unordered_map<std::string, const HipParamBinding*>& initSpec,
-                                     unsigned* gridOut, gdb_event beforeKernel, bool* marked) {
+                                     bool foldFollows, unsigned* gridOut, gdb_event beforeKernel, bool* marked) {
     std::vector<uint64_t> args;
     args.reserve(p.bindings.size());
     bool filled = false;
@@ -324,7 +324,10 @@ void HipGenericExecutor::launchPhase(RuntimeCompiler& rc, const RuntimeCompiler:
                 args.push_back(static_cast<uint64_t>(s->second));
                 break;
             }
-            case HipParamKind::SymbolValue: args.push_back(sizes_.resolve(b.sizeExpr)); break;
+            case HipParamKind::SymbolValue:
+                // partials that nothing folds would be missing from the result
+                args.push_back(!foldFollows && b.name == p.partialsSymbol ? 0 : sizes_.resolve(b.sizeExpr));
+                break;
         }
     }
     const int items = p.isSingleThread ? 1 : p.items;
@@ -455,7 +458,7 @@ void HipGenericExecutor::enqueue(RuntimeCompiler& rc, const RuntimeCompiler::Com
     std::unordered_map<std::string, bool> initDone;
     hoistInits(cg, firstPhase, last, initDone, spec);
     for (int pi = firstPhase; pi < last; ++pi)
-        launchPhase(rc, cq, phases[static_cast<size_t>(pi)], initDone, spec, nullptr, nullptr, nullptr);
+        launchPhase(rc, cq, phases[static_cast<size_t>(pi)], initDone, spec, true, nullptr, nullptr, nullptr);
 }
 
 HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq,
@@ -497,7 +500,10 @@ HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const Runtim
             unsigned grid = 0;
             const size_t e = static_cast<size_t>(2 * (pi - firstPhase));
             bool marked = apart;
-            launchPhase(rc, cq, p, initDone, spec, &grid, phaseTiming_ ? events_[e + 1] : nullptr, &marked);
+            bool foldFollows = p.partialsSymbol.empty() || p.foldsPartials;
+            for (int f = pi + 1; f < last; ++f)
+                foldFollows |= phases[static_cast<size_t>(f)].partialsSymbol == p.partialsSymbol;
+            launchPhase(rc, cq, p, initDone, spec, foldFollows, &grid, phaseTiming_ ? events_[e + 1] : nullptr, &marked);
             ownStart_[static_cast<size_t>(pi - firstPhase)] = marked;
             apart = false;
             if (phaseTiming_ || pi + 1 == last) check(gdb_event_record(events_[e + 2], stream_), "gdb_event_record");

@@ -91,10 +91,12 @@ public:
     // Allocate every buffer of phases [first, last) that can be sized now.
     void prepare(const HipCodegen& cg, int firstPhase = 0, int lastPhase = -1);
     // Launch phases [first, last) on the stream: init fills + kernels only.
-    // Hooks are ignored; no synchronisation.
+    // Hooks are ignored; no synchronisation. Partial tables are left for a fold
+    // phase that the caller runs, also outside the range (chunks of a table).
     void enqueue(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq, const HipCodegen& cg,
                  int firstPhase = 0, int lastPhase = -1);
-    // Warm up, then time `measured` runs (results of the last run remain).
+    // Warm up, then time `measured` runs (results of the last run remain). A
+    // scan whose fold phase is not in the range merges without partial tables.
     HipExecutionResult execute(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq, const HipCodegen& cg,
                                int warmupRuns = 0, int measuredRuns = 1, int firstPhase = 0, int lastPhase = -1);
     // Pieces of a launch, for callers that fuse phases of several plans into
@@ -234,7 +236,7 @@ private:
     void resolveBufferTables();
     void launchPhase(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq, const HipCodegen::PhaseInfo& p,
                      std::unordered_map<std::string, bool>& initDone, const std::unordered_map<std::string, const HipParamBinding*>& initSpec,
-                     unsigned* gridOut, gdb_event beforeKernel, bool* marked);
+                     bool foldFollows, unsigned* gridOut, gdb_event beforeKernel, bool* marked);
     // Buffers (and bytes) a small result of this schema reads.
     std::vector<std::pair<std::string, size_t>> resultBuffers(const HipResultSchema& rs) const;
     std::unordered_map<std::string, const HipParamBinding*> initSpecs(const HipCodegen& cg) const;

@@ -1812,10 +1812,11 @@ void HipHashGroupBy::produceImpl(HipCodegen& cg, ConsumerFn consume) {
             cg.addComment("the LDS table becomes partial table _pi, if one is left");
             cg.declareLds("u64", "_pti_" + T, "1");
             // a launch of a few blocks merges each key a few times: the fold
-            // would cost more than it saves (measured in the plan builder)
+            // would cost more than it saves (measured in the plan builder);
+            // no room for partials: no fold follows in this run
             const std::string take = "__hip_atomic_fetch_add(" + PN + ", 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)";
             cg.addLine("if (threadIdx.x == 0) _pti_" + T + "[0] = " +
-                       (cg.rangeMode() ? take : "gridDim.x < " + s(kMinFoldBlocks) + "u ? ~0ull : " + take) + ";");
+                       (cg.rangeMode() ? take : "gridDim.x < " + s(kMinFoldBlocks) + "u || " + NP + " == 0ull ? ~0ull : " + take) + ";");
             cg.addLine("__syncthreads();");
             cg.addLine("const u64 _pi_" + T + " = _pti_" + T + "[0];");
             cg.addBlock("if (_pi_" + T + " < " + NP + ")", [&]() {

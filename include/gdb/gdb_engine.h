@@ -126,7 +126,9 @@ typedef struct {
  * (codegen/execution/metal_generic_executor.cpp:289-399). */
 gdb_status gdb_executor_execute(gdb_executor ex, gdb_plan p, int warmup, int measured, gdb_exec_timing* out);
 /* Phases [first, last) only (last = -1: to the end). Replaces the
- * phase-range execute (metal_generic_executor.h:86-93). */
+ * phase-range execute (metal_generic_executor.h:86-93). A group-by scan whose
+ * fold phase lies outside the range leaves no partial tables: every block
+ * merges into the group table, which is complete behind the scan. */
 gdb_status gdb_executor_execute_range(gdb_executor ex, gdb_plan p, int first, int last, int warmup, int measured,
                                       gdb_exec_timing* out);
 /* Allocate, then launch without synchronising (graph capture, overlap). */

@@ -84,6 +84,39 @@ def test_fold_of_batched_pipelines(ctx, chunk, lds_bits):
         w.close()
 
 
+def test_scan_phase_alone_leaves_the_whole_table(ctx):
+    """Phase ranges: the scan without its fold, the fold after it on its own,
+    and both together hold every group once."""
+    G = _table(300_001, 900, 7)
+    dev = Q.upload_tables(ctx, {"G": G})
+    try:
+        run = Q.run_groupby(ctx, dev, slots=2048, variant="lds")
+        ex, plan = run.executor, run.plan
+        assert plan.phases() == ["GB_agg", "GB_merge"]
+        ex.execute(plan, first=0, last=1)
+        _same(ex.collect(plan).columns, G)
+        ex.execute(plan, first=1, last=2)
+        _same(ex.collect(plan).columns, G)
+        ex.execute(plan)
+        _same(ex.collect(plan).columns, G)
+    finally:
+        dev["G"].free(ctx)
+
+
+def test_pipeline_scan_alone_leaves_the_whole_table(ctx):
+    w = B.Workload3(ctx, B.workload3(n_pipes=8, scale=0.2, seed=78), lds_cap=4096, partials=32)
+    try:
+        w.run_plain()
+        plain = w.results()
+        for s in w.specs:
+            if s.kind == "agg":
+                w.execs[s.index].execute(w.batch_plans["agg"], first=0, last=1)
+        for got, exp in zip(w.results(), plain):
+            assert all(np.array_equal(got[k], exp[k]) for k in exp)
+    finally:
+        w.close()
+
+
 def _autotune(ex, plan, phase, blocks, items):
     bl, it = (C.c_int * len(blocks))(*blocks), (C.c_int * len(items))(*items)
     block, n, ms, count = C.c_int(), C.c_int(), C.c_float(), C.c_int()
