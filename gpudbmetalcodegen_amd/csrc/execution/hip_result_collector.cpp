@@ -117,12 +117,23 @@ void ResultColumn::copyI64(int64_t* out) const {
     // a thread costs ~20 us to start, 256K values ~0.5-1 ms to write to fresh pages
     const size_t threads = std::min<size_t>(8, rawRows / (1u << 18));
     if (threads < 2) return part(0, rawRows);
-    std::vector<std::thread> pool;
+    struct Pool {
+        std::vector<std::thread> t;
+        ~Pool() {
+            for (auto& th : t) th.join();
+        }
+    } pool;
+    pool.t.reserve(threads - 1);
     const size_t step = (rawRows + threads - 1) / threads;
-    for (size_t t = 1; t < threads; ++t)
-        pool.emplace_back(part, std::min(rawRows, t * step), std::min(rawRows, (t + 1) * step));
+    for (size_t t = 1; t < threads; ++t) {
+        const size_t b = std::min(rawRows, t * step), e = std::min(rawRows, (t + 1) * step);
+        try {
+            pool.t.emplace_back(part, b, e);
+        } catch (const std::exception&) {  // no thread to be had
+            part(b, e);
+        }
+    }
     part(0, step);
-    for (auto& th : pool) th.join();
 }
 
 const ResultColumn& GenericResult::column(const std::string& name) const {
