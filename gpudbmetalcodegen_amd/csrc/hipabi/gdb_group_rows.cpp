@@ -8,11 +8,11 @@
 
 #include "gdb/gdb_hip.h"
 #include "gdb/gdb_kernels.h"
+#include "gdb_error.h"
 
 #include <hip/hip_runtime.h>
-#include <algorithm>
 
-#include <string>
+#include <algorithm>
 
 namespace {
 
@@ -22,19 +22,7 @@ typedef unsigned long long u64;
 constexpr u32 kEmpty = 0xFFFFFFFFu;
 constexpr u32 kSmallRows = GDB_GROUP_ROWS_SMALL;
 
-thread_local std::string g_err;
-
-gdb_status bad(const char* m) {
-    g_err = m;
-    return GDB_ERR_INVALID;
-}
-
-gdb_status launched(const char* what) {
-    const hipError_t e = hipGetLastError();
-    if (e == hipSuccess) return GDB_OK;
-    g_err = std::string(what) + ": " + hipGetErrorString(e);
-    return GDB_ERR_HIP;
-}
+gdb_status bad(const char* m) { return gdbhip::fail(GDB_ERR_INVALID, m); }
 
 __device__ __forceinline__ u32 lane() { return threadIdx.x & 63u; }
 __device__ __forceinline__ u64 lanesBelow() { return (1ull << lane()) - 1ull; }
@@ -303,14 +291,12 @@ size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 extern "C" {
 
-const char* gdb_group_rows_last_error(void) { return g_err.c_str(); }
-
 gdb_status gdb_group_rows_small(const uint64_t* table, uint64_t slots, uint64_t* pinned_out, gdb_stream s) {
     if (!table || !pinned_out) return bad("gdb_group_rows_small: null argument");
     if (slots > 2 * (uint64_t)kSmallRows) return bad("gdb_group_rows_small: too many slots");
     hipLaunchKernelGGL(groupRowsSmallKernel, dim3(1), dim3(1024), 0, (hipStream_t)s, (const u64*)table, (u32)slots,
                        (u64*)pinned_out);
-    return launched("groupRowsSmallKernel");
+    return gdbhip::launchCheck("groupRowsSmallKernel");
 }
 
 gdb_status gdb_group_rows_small_many(const gdb_group_table* tables, int n, gdb_stream s) {
@@ -325,7 +311,7 @@ gdb_status gdb_group_rows_small_many(const gdb_group_table* tables, int n, gdb_s
         std::copy(tables + i, tables + i + m, all.t);
         hipLaunchKernelGGL(groupRowsSmallManyKernel, dim3((u32)m), dim3(1024), 0, (hipStream_t)s, all);
     }
-    return launched("groupRowsSmallManyKernel");
+    return gdbhip::launchCheck("groupRowsSmallManyKernel");
 }
 
 gdb_status gdb_group_rows_compact(const uint64_t* table, uint64_t slots, uint64_t* pairs, uint64_t* head, gdb_stream s) {
@@ -335,7 +321,7 @@ gdb_status gdb_group_rows_compact(const uint64_t* table, uint64_t slots, uint64_
     if (slots)
         hipLaunchKernelGGL(groupCompactKernel, dim3((u32)((slots + 8191) / 8192)), dim3(1024), 0, (hipStream_t)s,
                            (const u64*)table, (u64)slots, (u64*)pairs, (u64*)head);
-    return launched("groupCompactKernel");
+    return gdbhip::launchCheck("groupCompactKernel");
 }
 
 size_t gdb_group_rows_scratch_bytes(uint64_t n) {
@@ -364,7 +350,7 @@ gdb_status gdb_group_rows_sort(const uint64_t* table, uint64_t* pairs, uint64_t 
     }
     hipLaunchKernelGGL(groupColumnsKernel, dim3((u32)((n + 255) / 256)), dim3(256), 0, (hipStream_t)s, (const u64*)table,
                        (const u64*)a, (u64)n, key, count, (u64*)sum, (u64*)mn, (u64*)mx);
-    return launched("groupColumnsKernel");
+    return gdbhip::launchCheck("groupColumnsKernel");
 }
 
 }  // extern "C"

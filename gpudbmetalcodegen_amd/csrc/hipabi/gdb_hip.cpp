@@ -7,6 +7,7 @@
 // hashes the source, the options, the architecture and the hipRTC version.
 
 #include "gdb/gdb_hip.h"
+#include "gdb_error.h"
 
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
@@ -25,20 +26,23 @@
 #include <unordered_map>
 #include <vector>
 
-namespace {
+static thread_local std::string g_err;
 
-thread_local std::string g_err;
-
-gdb_status fail(gdb_status code, const std::string& msg) {
+gdb_status gdbhip::fail(gdb_status code, const std::string& msg) {
     g_err = msg;
     return code;
 }
 
-gdb_status hipFail(hipError_t e, const char* what) {
+gdb_status gdbhip::hipFail(hipError_t e, const char* what) {
     std::string m = std::string(what) + ": " + hipGetErrorName(e) + " (" + hipGetErrorString(e) + ")";
     (void)hipGetLastError();  // clear the sticky-free error state for the next call
     return fail(e == hipErrorOutOfMemory ? GDB_ERR_OOM : GDB_ERR_HIP, m);
 }
+
+namespace {
+
+using gdbhip::fail;
+using gdbhip::hipFail;
 
 #define GDB_HIP_TRY(call, what)                       \
     do {                                              \

@@ -7,6 +7,7 @@
 
 #include "gdb/gdb_hip.h"
 #include "gdb/gdb_kernels.h"
+#include "gdb_error.h"
 
 #include <hip/hip_runtime.h>
 
@@ -16,18 +17,8 @@
 
 namespace {
 
-thread_local std::string g_kerr;
-
-gdb_status kfail(gdb_status code, const std::string& m) {
-    g_kerr = m;
-    return code;
-}
-
-gdb_status launchCheck(const char* what) {
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return kfail(GDB_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
-    return GDB_OK;
-}
+using gdbhip::fail;
+using gdbhip::launchCheck;
 
 // ---------------------------------------------------------------------------
 // MLP 16 -> 64 -> 64 -> 1, ReLU, FP32. Parameter layout (floats):
@@ -264,15 +255,15 @@ hipError_t g_scratch_err[kMaxDevices] = {};
 gdb_status scratchFor(float** out) {
     int dev = -1;
     hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return kfail(GDB_ERR_HIP, std::string("hipGetDevice: ") + hipGetErrorString(e));
-    if (dev < 0 || dev >= kMaxDevices) return kfail(GDB_ERR_INVALID, "scratch: device index out of range");
+    if (e != hipSuccess) return fail(GDB_ERR_HIP, std::string("hipGetDevice: ") + hipGetErrorString(e));
+    if (dev < 0 || dev >= kMaxDevices) return fail(GDB_ERR_INVALID, "scratch: device index out of range");
     std::call_once(g_scratch_once[dev], [dev]() {
         void* p = nullptr;
         g_scratch_err[dev] = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (g_scratch_err[dev] == hipSuccess) g_scratch_ptr[dev] = static_cast<float*>(p);
     });
     if (g_scratch_err[dev] != hipSuccess || !g_scratch_ptr[dev])
-        return kfail(GDB_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(g_scratch_err[dev]));
+        return fail(GDB_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(g_scratch_err[dev]));
     *out = g_scratch_ptr[dev];
     return GDB_OK;
 }
@@ -287,10 +278,10 @@ unsigned gridFor(unsigned long long n, unsigned cap = 8192) {
 
 extern "C" {
 
-const char* gdb_kernels_last_error(void) { return g_kerr.c_str(); }
+const char* gdb_kernels_last_error(void) { return gdb_last_error(); }
 
 gdb_status gdb_mlp_forward(const float* params, const float* X, float* Y, int n, gdb_stream s) {
-    if (n < 0) return kfail(GDB_ERR_INVALID, "gdb_mlp_forward: negative batch");
+    if (n < 0) return fail(GDB_ERR_INVALID, "gdb_mlp_forward: negative batch");
     if (n == 0) return GDB_OK;
     hipLaunchKernelGGL(mlpForwardKernel, dim3((n + SPB - 1) / SPB), dim3(256), 0, (hipStream_t)s, params, X, Y, n);
     return launchCheck("mlpForwardKernel");
@@ -298,7 +289,7 @@ gdb_status gdb_mlp_forward(const float* params, const float* X, float* Y, int n,
 
 gdb_status gdb_mlp_backward(const float* params, const float* X, const float* T, float* G, float* L, int n,
                             float scale, gdb_stream s) {
-    if (n <= 0) return kfail(GDB_ERR_INVALID, "gdb_mlp_backward: empty batch");
+    if (n <= 0) return fail(GDB_ERR_INVALID, "gdb_mlp_backward: empty batch");
     hipLaunchKernelGGL(mlpBackwardKernel, dim3((n + SPB - 1) / SPB), dim3(256), 0, (hipStream_t)s, params, X, T, G,
                        L, n, scale);
     return launchCheck("mlpBackwardKernel");
@@ -306,7 +297,7 @@ gdb_status gdb_mlp_backward(const float* params, const float* X, const float* T,
 
 gdb_status gdb_mlp_reduce_adam(float* params, float* m, float* v, const float* G, float* grad, int n, int step,
                                float lr, float beta1, float beta2, float eps, gdb_stream s) {
-    if (n <= 0) return kfail(GDB_ERR_INVALID, "gdb_mlp_reduce_adam: empty batch");
+    if (n <= 0) return fail(GDB_ERR_INVALID, "gdb_mlp_reduce_adam: empty batch");
     const float c1 = 1.0f - std::pow(beta1, (float)step);
     const float c2 = 1.0f - std::pow(beta2, (float)step);
     hipLaunchKernelGGL(mlpReduceAdamKernel, dim3((NP + 255) / 256), dim3(256), 0, (hipStream_t)s, params, m, v, G,
@@ -317,13 +308,13 @@ gdb_status gdb_mlp_reduce_adam(float* params, float* m, float* v, const float* G
 gdb_status gdb_mlp_train_step_noalloc(float* params, float* m, float* v, const float* X, const float* T, float* L,
                                      float* grad, int n, float scale, int step, float lr, float beta1, float beta2,
                                      float eps, gdb_stream s) {
-    if (n <= 0) return kfail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: empty batch");
+    if (n <= 0) return fail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: empty batch");
     if (n > GDB_MLP_NOALLOC_MAX_SAMPLES)
-        return kfail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: batch of " + std::to_string(n) +
+        return fail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: batch of " + std::to_string(n) +
                                           " samples exceeds the static workspace (" +
                                           std::to_string(GDB_MLP_NOALLOC_MAX_SAMPLES) + " samples)");
-    if (!params || !X || !T || !L) return kfail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: null argument");
-    if (lr > 0.0f && (!m || !v)) return kfail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: Adam moments missing");
+    if (!params || !X || !T || !L) return fail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: null argument");
+    if (lr > 0.0f && (!m || !v)) return fail(GDB_ERR_INVALID, "gdb_mlp_train_step_noalloc: Adam moments missing");
     float* G = nullptr;
     const gdb_status st = scratchFor(&G);
     if (st != GDB_OK) return st;
@@ -340,7 +331,7 @@ gdb_status gdb_mlp_train_step_noalloc(float* params, float* m, float* v, const f
 }
 
 gdb_status gdb_gen_device_zipf_i32(int32_t* out, uint64_t n, double s, int64_t nkeys, uint64_t seed, gdb_stream st) {
-    if (nkeys < 1 || s < 0.0) return kfail(GDB_ERR_INVALID, "gdb_gen_device_zipf_i32: bad parameters");
+    if (nkeys < 1 || s < 0.0) return fail(GDB_ERR_INVALID, "gdb_gen_device_zipf_i32: bad parameters");
     if (n == 0) return GDB_OK;
     hipLaunchKernelGGL(zipfKernel, dim3(gridFor(n)), dim3(256), 0, (hipStream_t)st, out, (unsigned long long)n, s,
                        (double)nkeys, (unsigned long long)seed);
@@ -348,7 +339,7 @@ gdb_status gdb_gen_device_zipf_i32(int32_t* out, uint64_t n, double s, int64_t n
 }
 
 gdb_status gdb_gen_device_uniform_i64(int64_t* out, uint64_t n, int64_t lo, int64_t hi, uint64_t seed, gdb_stream st) {
-    if (hi < lo) return kfail(GDB_ERR_INVALID, "gdb_gen_device_uniform_i64: hi < lo");
+    if (hi < lo) return fail(GDB_ERR_INVALID, "gdb_gen_device_uniform_i64: hi < lo");
     if (n == 0) return GDB_OK;
     hipLaunchKernelGGL(uniformI64Kernel, dim3(gridFor(n)), dim3(256), 0, (hipStream_t)st, (long long*)out,
                        (unsigned long long)n, (long long)lo, (long long)hi, (unsigned long long)seed);
@@ -356,10 +347,10 @@ gdb_status gdb_gen_device_uniform_i64(int64_t* out, uint64_t n, int64_t lo, int6
 }
 
 gdb_status gdb_gather_words(const uint64_t* const* src, int n, int words, uint64_t* dst, gdb_stream st) {
-    if (n < 0 || words < 1 || (n && (!src || !dst))) return kfail(GDB_ERR_INVALID, "gdb_gather_words: bad arguments");
+    if (n < 0 || words < 1 || (n && (!src || !dst))) return fail(GDB_ERR_INVALID, "gdb_gather_words: bad arguments");
     if (n == 0) return GDB_OK;
     const long long total = (long long)n * words;
-    if (total > (1ll << 30)) return kfail(GDB_ERR_INVALID, "gdb_gather_words: too many words");
+    if (total > (1ll << 30)) return fail(GDB_ERR_INVALID, "gdb_gather_words: too many words");
     hipLaunchKernelGGL(gatherWordsKernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)st,
                        (const unsigned long long* const*)src, n, words, (unsigned long long*)dst);
     return launchCheck("gatherWordsKernel");
@@ -367,12 +358,12 @@ gdb_status gdb_gather_words(const uint64_t* const* src, int n, int words, uint64
 
 gdb_status gdb_gather_to_host(const gdb_gather_piece* pieces, int n, void* pinned_dst, gdb_stream st) {
     if (n < 0 || n > GDB_GATHER_MAX || (n && (!pieces || !pinned_dst)))
-        return kfail(GDB_ERR_INVALID, "gdb_gather_to_host: bad arguments");
+        return fail(GDB_ERR_INVALID, "gdb_gather_to_host: bad arguments");
     if (n == 0) return GDB_OK;
     GatherList list;
     for (int i = 0; i < n; ++i) {
         if (!pieces[i].src || pieces[i].bytes % 4 || pieces[i].host_offset % 4)
-            return kfail(GDB_ERR_INVALID, "gdb_gather_to_host: pieces are 4-byte multiples");
+            return fail(GDB_ERR_INVALID, "gdb_gather_to_host: pieces are 4-byte multiples");
         list.piece[i] = pieces[i];
     }
     hipLaunchKernelGGL(gatherToHostKernel, dim3((unsigned)n), dim3(64), 0, (hipStream_t)st, list, (char*)pinned_dst);
@@ -381,7 +372,7 @@ gdb_status gdb_gather_to_host(const gdb_gather_piece* pieces, int n, void* pinne
 
 gdb_status gdb_copy_async(void* dst, const void* src, size_t bytes, gdb_stream st) {
     if (bytes % 16 || ((uintptr_t)dst % 16) || ((uintptr_t)src % 16))
-        return kfail(GDB_ERR_INVALID, "gdb_copy_async: 16-byte aligned sizes and pointers only");
+        return fail(GDB_ERR_INVALID, "gdb_copy_async: 16-byte aligned sizes and pointers only");
     if (!bytes) return GDB_OK;
     const unsigned long long n16 = bytes / 16;
     hipLaunchKernelGGL(copyKernel, dim3(gridFor(n16, 16384)), dim3(256), 0, (hipStream_t)st, (uint4*)dst,

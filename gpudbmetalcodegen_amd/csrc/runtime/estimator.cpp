@@ -22,11 +22,7 @@ namespace runtime {
 namespace {
 
 void check(gdb_status st, const char* what) {
-    if (st != GDB_OK) {
-        const char* m = gdb_last_error();
-        if (!m || !*m) m = gdb_kernels_last_error();
-        throw std::runtime_error(std::string(what) + ": " + (m ? m : ""));
-    }
+    if (st != GDB_OK) throw std::runtime_error(std::string(what) + ": " + gdb_last_error());
 }
 
 double lg2(double x) { return std::log2(std::max(1.0, x)); }

@@ -25,7 +25,7 @@ extern "C" {
 #define GDB_MLP_HIDDEN 64
 #define GDB_MLP_NPARAMS 5313 /* W1 64x16, b1 64, W2 64x64, b2 64, W3 64, b3 1 */
 
-const char* gdb_kernels_last_error(void);
+const char* gdb_kernels_last_error(void); /* the same text as gdb_last_error() */
 
 /* Y[s] = MLP(params, X[s][0..15]) for s < n. */
 gdb_status gdb_mlp_forward(const float* params, const float* X, float* Y, int n, gdb_stream s);
@@ -92,7 +92,6 @@ gdb_status gdb_gather_to_host(const gdb_gather_piece* pieces, int n, void* pinne
  * gdb_group_rows_scratch_bytes(n) of scratch) and writes n-element columns. */
 #define GDB_GROUP_ROWS_SMALL 8192
 #define GDB_GROUP_ROWS_SMALL_BYTES ((8 + 4 * GDB_GROUP_ROWS_SMALL) * 8)
-const char* gdb_group_rows_last_error(void);
 gdb_status gdb_group_rows_small(const uint64_t* table, uint64_t slots, uint64_t* pinned_out, gdb_stream s);
 /* The same for any number of tables, one block each and GDB_GROUP_MANY of
  * them a launch. */

@@ -121,6 +121,17 @@ def test_hiprtc_compile_error_surfaces_log(tmp_path):
     assert "undefined_name" in msg and "1: extern" in msg   # numbered source dump
 
 
+def test_error_text_is_that_of_the_last_failure(tmp_path):
+    """Every file of the library sets the text that gdb_last_error returns."""
+    hip, _ = N.load()
+    assert hip.gdb_group_rows_small(None, C.c_uint64(64), None, None) == N.GDB_ERR_INVALID
+    assert b"gdb_group_rows_small" in hip.gdb_last_error()
+    assert hip.gdb_gather_to_host(None, 1, None, None) == N.GDB_ERR_INVALID
+    assert b"gdb_gather_to_host" in hip.gdb_last_error()
+    assert hip.gdb_group_rows_compact(None, C.c_uint64(64), None, None, None) == N.GDB_ERR_INVALID
+    assert b"gdb_group_rows_compact" in hip.gdb_last_error() and hip.gdb_last_error() == hip.gdb_kernels_last_error()
+
+
 def test_plan_hash_depends_on_source_and_options(tmp_path):
     hip, _ = N.load()
     src = b'extern "C" __global__ void k(int* p) { p[0] = 1; }'
