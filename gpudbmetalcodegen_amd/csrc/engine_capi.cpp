@@ -222,22 +222,32 @@ gdb_status gdb_plan_phase_name(gdb_plan p, int idx, char* buf, size_t cap) {
     });
 }
 
+// Sets a phase's block and ITEMS; a block that needs another launch bound has
+// the plan generated again, and compiled if it was.
+static void setPhaseLaunch(gdb_plan p, size_t idx, int block, int items) {
+    auto& own = p->plan.phases[idx];
+    auto& ph = p->cg.getPhasesMutable()[idx];
+    own.threadgroupSize = ph.threadgroupSize = block;
+    own.items = ph.items = items;
+    if (own.bound() == ph.launchBound) return;
+    const bool compiled = p->compiled;
+    p->regenerate();
+    if (!compiled) return;
+    p->cq = compilerFor(p->ctx).compile(p->source);
+    p->compiled = true;
+}
+
 gdb_status gdb_plan_set_launch(gdb_plan p, const char* phase, int block, int items) {
     return guard([&]() -> gdb_status {
-        for (auto& ph : p->cg.getPhasesMutable()) {
+        const auto& phases = p->plan.phases;
+        for (size_t i = 0; i < phases.size(); ++i) {
+            const auto& ph = phases[i];
             if (ph.name != phase) continue;
-            bool known = false;
-            for (int v : ph.itemsVariants) known |= (v == items);
-            if (!known) return setErr(GDB_ERR_INVALID, "gdb_plan_set_launch: no ITEMS variant " + std::to_string(items));
-            if (block < 64 || block > ph.launchBound || block % 64)
+            if (std::find(ph.itemsVariants.begin(), ph.itemsVariants.end(), items) == ph.itemsVariants.end())
+                return setErr(GDB_ERR_INVALID, "gdb_plan_set_launch: no ITEMS variant " + std::to_string(items));
+            if (block < 64 || block > std::max(ph.launchBound, ph.maxBlock) || block % 64)
                 return setErr(GDB_ERR_INVALID, "gdb_plan_set_launch: block size outside [64, launch bound]");
-            ph.threadgroupSize = block;
-            ph.items = items;
-            for (auto& pp : p->plan.phases)
-                if (pp.name == phase) {
-                    pp.threadgroupSize = block;
-                    pp.items = items;
-                }
+            setPhaseLaunch(p, i, block, items);
             return GDB_OK;
         }
         return setErr(GDB_ERR_NOT_FOUND, std::string("gdb_plan_set_launch: no phase ") + phase);
@@ -737,17 +747,32 @@ gdb_status gdb_autotune_phase(gdb_executor ex, gdb_plan p, const char* phase, co
         if (idx < 0) return setErr(GDB_ERR_NOT_FOUND, std::string("gdb_autotune_phase: no phase ") + phase);
         registerPlanTables(ex, p);
         ex->ex->clearPhaseHooks();
-        auto r = runtime::autotunePhase(*ex->ex, compilerFor(ex->ctx), p->cq, p->cg, idx,
-                                        std::vector<int>(blocks, blocks + nblocks), std::vector<int>(items, items + nitems),
-                                        scalar_name ? scalar_name : "",
-                                        std::vector<int64_t>(scalar_values, scalar_values + (scalar_values ? nscalars : 0)),
-                                        trials);
+        const size_t at = static_cast<size_t>(idx);
+        const std::string scalar = scalar_name ? scalar_name : "";
+        auto tune = [&](const std::vector<int>& bl) {
+            return runtime::autotunePhase(*ex->ex, compilerFor(ex->ctx), p->cq, p->cg, idx, bl,
+                                          std::vector<int>(items, items + nitems), scalar,
+                                          std::vector<int64_t>(scalar_values, scalar_values + (scalar_values ? nscalars : 0)),
+                                          trials);
+        };
+        const auto& own = p->plan.phases[at];
+        const int block0 = own.threadgroupSize, items0 = own.items;
+        std::vector<int> within, beyond;  // blocks within the launch bound; blocks the phase is generated for one by one
+        for (int k = 0; k < nblocks; ++k)
+            (blocks[k] > own.launchBound && blocks[k] <= own.maxBlock && blocks[k] % 64 == 0 ? beyond : within).push_back(blocks[k]);
+        if (!beyond.empty() && block0 > own.launchBound) setPhaseLaunch(p, at, own.launchBound, items0);
+        auto r = tune(within);
+        for (int b : beyond) {
+            setPhaseLaunch(p, at, b, items0);
+            auto q = tune({b});
+            auto table = std::move(r.table);
+            table.insert(table.end(), q.table.begin(), q.table.end());
+            if (q.block && (!r.block || q.ms < r.ms)) r = q;
+            r.table = std::move(table);
+        }
+        setPhaseLaunch(p, at, r.block ? r.block : block0, r.block ? r.items : items0);
+        if (!scalar.empty() && r.block) ex->ex->registerScalarInt(scalar, r.scalar);
         if (r.block == 0) return setErr(GDB_ERR_INVALID, "gdb_autotune_phase: no candidate ran");
-        for (auto& pp : p->plan.phases)
-            if (pp.name == phase) {
-                pp.threadgroupSize = r.block;
-                pp.items = r.items;
-            }
         if (best_block) *best_block = r.block;
         if (best_items) *best_items = r.items;
         if (best_scalar) *best_scalar = r.scalar;

@@ -215,7 +215,10 @@ HipQueryPlan buildQ3(const PlanOptions& o) {
         // together (without the queue): 0.177 ms at 15M rows, where ~10% of
         // the rows reach the CAS and a batch rarely holds more than one
         ph.staged = compactB || optInt(o, "staged", 0) != 0;
-        if (compactB) ph.launchBound = blockB;  // sizes the per-wave queues
+        if (compactB) {
+            ph.launchBound = blockB;  // sizes the per-wave queues: at 1024 three blocks of 512 a CU, not four
+            ph.maxBlock = 1024;
+        }
         ph.prefetch = optInt(o, "prefetch", 0) != 0;
     }
     if (probeBitmap && bflags) {
@@ -285,7 +288,7 @@ HipQueryPlan buildQ3(const PlanOptions& o) {
         // threads, inserting candidates one by one: 16-19 us; now 11-12)
         const int mergeBlock = optInt(o, "merge_block", HipTopK::kMaxBlocks);
         auto& pm = appendPhase(plan, "Q3_topk_merge", std::move(merge), mergeBlock, 1, {1});
-        pm.launchBound = std::max<int>(HipTopK::kMaxBlocks, mergeBlock);
+        pm.launchBound = 1024;
     }
     plan.requiredScalars = {"q3_seg", "q3_date"};
     plan.requiredSymbols = {"a_bits", "b_bits"};
@@ -699,7 +702,7 @@ HipCodegen generateFromPlan(const HipQueryPlan& plan, bool rangeMode) {
         cg.setPhaseSingleThread(phase.singleThread);
         cg.setPhaseItemsVariants(phase.itemsVariants);
         cg.setPhaseItems(phase.items);
-        cg.setPhaseLaunchBound(phase.launchBound);
+        cg.setPhaseLaunchBound(phase.bound());
         cg.setPhaseStaged(phase.staged);
         cg.setPhasePrefetch(phase.prefetch);
         if (phase.maxThreadgroups) cg.setPhaseMaxThreadgroups(phase.maxThreadgroups);

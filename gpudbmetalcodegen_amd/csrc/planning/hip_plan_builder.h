@@ -12,6 +12,7 @@
 
 #include "../operators/hip_operators.h"
 
+#include <algorithm>
 #include <map>
 #include <memory>
 #include <optional>
@@ -31,6 +32,10 @@ struct HipQueryPlan {
         int items = 4;
         std::vector<int> itemsVariants{4};
         int launchBound = 1024;
+        // Largest block the phase may be set to (0: the launch bound); with a
+        // block above the launch bound it is generated with that as its bound.
+        int maxBlock = 0;
+        int bound() const { return std::max(launchBound, std::min(threadgroupSize, maxBlock)); }
         int maxThreadgroups = 0;
         bool singleThread = false;
         // Item-batched emission: the random loads (bitmap words, first hash

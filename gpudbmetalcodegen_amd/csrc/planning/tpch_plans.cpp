@@ -125,7 +125,7 @@ HipQueryPlan tpchQ3(const PlanOptions& o) {
         // threads, inserting candidates one by one: 16-19 us; now 11-12)
         const int mergeBlock = optInt(o, "merge_block", HipTopK::kMaxBlocks);
         auto& pm = appendPhase(plan, "Q3_topk_merge", std::move(merge), mergeBlock, 1, {1});
-        pm.launchBound = std::max<int>(HipTopK::kMaxBlocks, mergeBlock);
+        pm.launchBound = 1024;
     }
     plan.requiredScalars = {"q3_seg", "q3_date"};
     plan.requiredSymbols = {"c_bits", "o_bits", "o_slots"};

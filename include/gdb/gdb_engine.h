@@ -78,7 +78,8 @@ gdb_status gdb_plan_phase_count(gdb_plan p, int* n);
 gdb_status gdb_plan_phase_name(gdb_plan p, int idx, char* buf, size_t cap);
 /* Launch configuration of one phase (block size, ITEMS variant); the
  * reference's getPhasesMutable() used by --autotune-tg
- * (codegen/codegen_main.cpp:837-929). */
+ * (codegen/codegen_main.cpp:837-929). A phase whose queues are sized by its
+ * launch bound is generated and compiled again for a block above the bound. */
 gdb_status gdb_plan_set_launch(gdb_plan p, const char* phase, int block, int items);
 gdb_status gdb_plan_get_launch(gdb_plan p, const char* phase, int* block, int* items);
 /* Compile through the context's RuntimeCompiler (hipRTC + plan-hash cache).

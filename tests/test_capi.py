@@ -121,6 +121,27 @@ def test_hiprtc_compile_error_surfaces_log(tmp_path):
     assert "undefined_name" in msg and "1: extern" in msg   # numbered source dump
 
 
+def test_set_launch_up_to_1024_threads():
+    """Blocks above the default one: the queued join build is generated again
+    with that launch bound, and as before when set back."""
+    for opts, merge in (("", "Q3_topk_merge"), ("block_b=256", "Q3_topk_merge"), ("merge_block=64", "Q3_topk_merge"),
+                        ("schema=tpch", "Q3_topk_merge")):
+        p = E.build_hip_plan("Q3", opts)
+        p.set_launch(merge, 1024, 1)
+        assert p.get_launch(merge) == (1024, 1)
+        if "tpch" in opts:
+            continue
+        source, shape = p.source(), p.get_launch("Q3_build_b_table")
+        for block in (512, 1024):
+            p.set_launch("Q3_build_b_table", block, shape[1])
+            assert p.get_launch("Q3_build_b_table") == (block, shape[1]) and p.get_launch(merge) == (1024, 1)
+            assert f"__launch_bounds__({block}) Q3_build_b_table" in p.source()
+        with pytest.raises(N.GdbError):
+            p.set_launch("Q3_build_b_table", 1088, shape[1])
+        p.set_launch("Q3_build_b_table", *shape)
+        assert p.source() == source
+
+
 def test_error_text_is_that_of_the_last_failure(tmp_path):
     """Every file of the library sets the text that gdb_last_error returns."""
     hip, _ = N.load()
