@@ -755,11 +755,12 @@ std::vector<HipGenericExecutor::Piece> HipGenericExecutor::resultPieces(const Hi
                                                                         size_t* total) const {
     std::vector<Piece> have;
     for (const auto& b : resultBuffers(schema)) {
-        auto it = buffers_.find(b.first);
+        auto it = buffers_.find(b.name);
         if (it == buffers_.end()) continue;
-        const size_t bytes = std::min({b.second, it->second.bytes, size_t{16384}}) / 4 * 4;
+        if (b.whole && b.bytes > kMaxPiece) continue;  // one read, of more than the piece could hold
+        const size_t bytes = std::min({b.bytes, it->second.bytes, kMaxPiece}) / 4 * 4;
         if (bytes == 0) continue;
-        have.push_back({b.first, bytes, *total});
+        have.push_back({b.name, bytes, *total});
         *total += (bytes + 15) / 16 * 16;
     }
     return have;
@@ -851,17 +852,17 @@ std::vector<GenericResult> HipGenericExecutor::collectMany(
     return res;
 }
 
-std::vector<std::pair<std::string, size_t>> HipGenericExecutor::resultBuffers(const HipResultSchema& rs) const {
+std::vector<HipGenericExecutor::ResultRead> HipGenericExecutor::resultBuffers(const HipResultSchema& rs) const {
     switch (rs.kind) {
         case HipResultSchema::KEYED_AGG:
-            return {{rs.keyed.bufferName, static_cast<size_t>(rs.keyed.numBuckets) * static_cast<size_t>(rs.keyed.wordsPerBucket) * 8}};
+            return {{rs.keyed.bufferName, static_cast<size_t>(rs.keyed.numBuckets) * static_cast<size_t>(rs.keyed.wordsPerBucket) * 8, true}};
         case HipResultSchema::TOPK:
-            return {{rs.topk.ctlBuffer, 32}, {rs.topk.bufferName, 16 * static_cast<size_t>(rs.topk.k)}};
+            return {{rs.topk.ctlBuffer, 32, true}, {rs.topk.bufferName, 16 * static_cast<size_t>(rs.topk.k), true}};
         case HipResultSchema::HISTOGRAM:
         case HipResultSchema::COUNTS:
-            return {{rs.counts.bufferName, static_cast<size_t>(sizes_.resolve(rs.counts.sizeExpr)) * 4}};
+            return {{rs.counts.bufferName, static_cast<size_t>(sizes_.resolve(rs.counts.sizeExpr)) * 4, true}};
         case HipResultSchema::ROWS:
-            return {{rs.rows.ctlBuffer, 32}, {rs.rows.bufferName, rs.rows.fields.size() * 8 * 64}};  // the first 64 rows
+            return {{rs.rows.ctlBuffer, 32, true}, {rs.rows.bufferName, rs.rows.fields.size() * 8 * 64, false}};  // the first 64 rows
         default: return {};
     }
 }

@@ -218,6 +218,7 @@ private:
     bool collectGroups(const HipResultSchema& schema, GenericResult& res);
     const uint64_t* groupTable(const HipResultSchema& schema, uint64_t* slots) const;  // null: the host reads the table
     static bool smallGroups(const HipResultSchema& schema, const uint64_t* w, GenericResult& res);
+    static constexpr size_t kMaxPiece = 16384;
     struct Piece {  // the start of a result buffer, read to the host at `at`
         std::string name;
         size_t bytes = 0, at = 0;
@@ -237,8 +238,14 @@ private:
     void launchPhase(RuntimeCompiler& rc, const RuntimeCompiler::CompiledQuery& cq, const HipCodegen::PhaseInfo& p,
                      std::unordered_map<std::string, bool>& initDone, const std::unordered_map<std::string, const HipParamBinding*>& initSpec,
                      bool foldFollows, unsigned* gridOut, gdb_event beforeKernel, bool* marked);
-    // Buffers (and bytes) a small result of this schema reads.
-    std::vector<std::pair<std::string, size_t>> resultBuffers(const HipResultSchema& rs) const;
+    // Buffers (and bytes) a result of this schema reads; whole: with one read
+    // of all those bytes, otherwise of as many as there are rows.
+    struct ResultRead {
+        std::string name;
+        size_t bytes;
+        bool whole;
+    };
+    std::vector<ResultRead> resultBuffers(const HipResultSchema& rs) const;
     std::unordered_map<std::string, const HipParamBinding*> initSpecs(const HipCodegen& cg) const;
     // Initialise, in one launch, every buffer defined by phases [first, last)
     // whose size is known now; marks them done.

@@ -47,6 +47,18 @@ def test_named_plans_text(ctx):
         db.free()
 
 
+@pytest.mark.parametrize("bins", [5, 4095, 4096, 4097, 9000])
+def test_counts_around_the_largest_piece(ctx, bins):
+    """Histograms read with the run's other words, and beyond 16 KB by a copy."""
+    db = T.TpchDB(ctx, G.generate(0.01, seed=3))
+    try:
+        res, exp = T.run(ctx, db, "Q13", options=f"hist_bins={bins}").raw, T.run(ctx, db, "Q13").raw
+        rows = [(c, n) for c, n in zip(exp.columns["c_count"], exp.columns["custdist"]) if c < bins]
+        assert list(zip(res.columns["c_count"], res.columns["custdist"])) == rows and res.canonical == _text(res)
+    finally:
+        db.free()
+
+
 def test_scan_text_and_no_rows(ctx):
     dev = Q.upload_tables(ctx, W.workload0(5000))
     try:
