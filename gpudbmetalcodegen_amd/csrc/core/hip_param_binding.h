@@ -42,6 +42,9 @@ inline std::string tableDataName(const std::string& table, const std::string& co
     return "p_" + col;
 }
 inline std::string tableSizeName(const std::string& table) { return "n_" + table; }
+// Most rows a table has been registered with: the whole table's while a chunk
+// of it is.
+inline std::string tableMaxSizeName(const std::string& table) { return "nmax_" + table; }
 
 struct HipParamBinding {
     std::string name;          // parameter name inside the kernel

@@ -67,6 +67,9 @@ void HipGenericExecutor::syncStream() {
 void HipGenericExecutor::registerTable(const std::string& table, uint64_t rows) {
     tables_[table].rows = rows;
     sizes_.registerSymbol(tableSizeName(table), rows);
+    uint64_t most = 0;
+    tryGetSymbol(tableMaxSizeName(table), most);
+    sizes_.registerSymbol(tableMaxSizeName(table), std::max(most, rows));
 }
 
 void HipGenericExecutor::registerTableColumn(const std::string& table, const std::string& column, const void* devptr) {

@@ -1863,7 +1863,7 @@ void HipGroupByMerge::produceImpl(HipCodegen& cg, ConsumerFn consume) {
     cg.addBufferParam(PN, "u64", 8, "2", InitKind::Zero, {}, false, true);
     cg.addSymbolParam(NP, partialsMax_);
     cg.setPhasePartials(NP, true);
-    cg.setPhaseRowsExpr("(" + partialsMax_ + ") * " + CAP);
+    cg.setPhaseRowsExpr(rows_.empty() ? "(" + partialsMax_ + ") * " + CAP : rows_);
     cg.addComment("GroupByMerge " + T + ": a block takes a range of home slots over every partial table, so each key "
                   "reaches the global table once");
     cg.declareLds("u64", tab, CAP + " * 4");

@@ -694,6 +694,8 @@ public:
         : table_(table), slots_(slotsExpr), ldsSlots_(ldsSlots), partialsMax_(partialsMax) {}
     void setRuntimeLdsBits(const std::string& scalarName) { ldsBitsScalar_ = scalarName; }
     void setWindow(int window) { window_ = window; }  // the scan's probe window
+    // Rows that size the grid where they are not the partials' (plain launches).
+    void setRows(const std::string& expr) { rows_ = expr; }
     void produceImpl(HipCodegen& cg, ConsumerFn consume) override;
     std::string describe() const override;
 
@@ -702,7 +704,7 @@ private:
     std::string table_, slots_;
     int ldsSlots_;
     int window_ = 16;
-    std::string partialsMax_, ldsBitsScalar_;
+    std::string partialsMax_, ldsBitsScalar_, rows_;
 };
 
 // Partitioned hash group-by: no counterpart in the reference, whose

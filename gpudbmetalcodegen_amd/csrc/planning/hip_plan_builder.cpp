@@ -390,13 +390,16 @@ HipQueryPlan buildGroupBy(const PlanOptions& o) {
     // LDS variant: the blocks' LDS tables are folded by GB_merge instead of
     // merged into the group table one by one, which cost the same keys' four
     // atomics once per block, all on the same lines: 1M rows of 700 groups
-    // took 353 us so, 16 us and a fold of 20 us now. As many partial tables as blocks can
-    // run at once (one per 32 B x lds_slots of a CU's 160 KB, 256 CUs), whatever
-    // the rows, so a chunked run keeps what earlier chunks left. Below 16
-    // blocks there is little to fold and they merge directly.
+    // took 353 us so, 16 us and a fold of 20 us now. As many partial tables as
+    // blocks can run at once (one per 32 B x lds_slots of a CU's 160 KB, 256
+    // CUs: 33.5 MB at 2,048 slots), and no more than the whole table makes
+    // blocks of 64 x 4 rows; a chunked run, which folds behind its last chunk,
+    // keeps what earlier chunks left. Below 16 blocks there is little to fold
+    // and they merge directly.
     const bool fold = variant == "lds";
     const int perCu = std::max(1, std::min(4, 155 * 1024 / (32 * ldsSlots)));
-    const std::string pmax = std::to_string(256 * perCu);
+    const std::string running = std::to_string(256 * perCu);
+    const std::string pmax = "min(" + running + ", " + tableMaxSizeName("G") + " / 256 + 1)";
     if (fold) gb->setPartials(pmax);
     // block 1024: as many waves per CU as two blocks of 512, half the partials
     // (100M rows 454 us against 556 at 512; 1M 18 us and a fold of 21, against 20 and 32)
@@ -409,6 +412,8 @@ HipQueryPlan buildGroupBy(const PlanOptions& o) {
     if (fold) {
         auto mg = std::make_unique<HipGroupByMerge>("d_gb_ht", "gb_slots", ldsSlots, pmax);
         mg->setWindow(optInt(o, "window", 16));
+        // the fold's blocks share the home slots, however few the partials
+        mg->setRows(running + " * " + std::to_string(ldsSlots));
         auto& pm = appendPhase(plan, "GB_merge", std::move(mg), 1024, 16, {16});
         pm.launchBound = 1024;
     }

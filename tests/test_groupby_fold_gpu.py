@@ -51,6 +51,23 @@ def test_fold_matches_oracle(ctx, lds_slots, n, groups, skew):
         dev["G"].free(ctx)
 
 
+def test_partial_tables_take_the_room_the_rows_need(ctx):
+    """A small table's runner holds little; the same runner then serves a larger
+    table, and again the small one."""
+    small, large = _table(1000, 300, 3), _table(300_001, 900, 4)
+    dev = Q.upload_tables(ctx, {"G": small}), Q.upload_tables(ctx, {"G": large})
+    try:
+        run = Q.run_groupby(ctx, dev[0], slots=2048, variant="lds")
+        _same(run.result.columns, small)
+        assert run.executor.owned_bytes() < 1 << 20
+        for k, G in ((1, large), (0, small)):
+            again = Q.run_groupby(ctx, dev[k], slots=2048, variant="lds", executor=run.executor)
+            _same(again.result.columns, G)
+    finally:
+        for d in dev:
+            d["G"].free(ctx)
+
+
 def test_fold_of_a_chunked_run(ctx):
     G = _table(500_000, 700, 5)
     h = E.HostTable("G", G)
