@@ -18,14 +18,18 @@ pytestmark = pytest.mark.gpu
 
 def _groups(ctx, n, slots, stream=None):
     r = np.random.default_rng(n + slots)
-    G = {"g_key": r.permutation(np.arange(n, dtype=np.int32) * 5 + 1), "g_val": r.integers(-10**9, 10**9, n)}
+    rows = max(n, 100)
+    G = {"g_key": r.permutation(np.arange(rows, dtype=np.int32) * 5 + 1), "g_val": r.integers(-10**9, 10**9, rows)}
     dev = Q.upload_tables(ctx, {"G": G})
-    run = Q.run_groupby(ctx, dev, slots=slots, variant="global", executor=E.HipGenericExecutor(ctx, stream))
+    cut = None if n == rows else int(np.sort(G["g_val"])[n])   # n rows pass
+    run = Q.run_groupby(ctx, dev, slots=slots, variant="global", val_cut=cut, executor=E.HipGenericExecutor(ctx, stream))
+    assert run.result.rows() == n
     return run, dev
 
 
-# 0 groups (every row cut), the one-block form's ends, the general path, and 70 tables (two launches)
-@pytest.mark.parametrize("sizes", [[], [(1, 64)], [(700, 2048)] * 3, [(8192, 16384), (8193, 16384), (20_000, 65536), (63, 128)],
+# no runner, 0 groups (every row cut) in the one-block form and the general path, the one-block form's ends, the
+# general path, and 70 tables (two launches)
+@pytest.mark.parametrize("sizes", [[], [(0, 64), (5, 64), (0, 65536)], [(1, 64)], [(700, 2048)] * 3, [(8192, 16384), (8193, 16384), (20_000, 65536), (63, 128)],
                                    [(10 + i, 64 + 64 * (i % 2)) for i in range(70)]])
 def test_group_tables(ctx, sizes):
     made = [_groups(ctx, n, slots) for n, slots in sizes]

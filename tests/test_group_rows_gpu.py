@@ -2,9 +2,12 @@
 device (the result of every group-by): against a sort at the sizes where
 the one-block form, the sort's tiles and its digit passes end."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from gpudbmetalcodegen_amd import _native as N
 from gpudbmetalcodegen_amd import queries as Q
 from helpers import group_rows
 
@@ -44,17 +47,37 @@ def test_key_ranges(ctx, top):
     _check(ctx, keys, 1 << 16)
 
 
-def test_large_result_is_held_apart_from_the_next(ctx):
-    n = 600_000
+# the general path's result lives in page-locked memory of the runner; the one-block form's is copied
+@pytest.mark.parametrize("n,slots", [(600_000, 1_200_000), (5000, 16384)])
+def test_result_is_held_apart_from_the_next(ctx, n, slots):
+    """A result that is still open keeps its values while the same runner
+    collects others, is released and is closed."""
+    eng = N.load()[1]
     G = {"g_key": np.random.default_rng(3).permutation(n).astype(np.int32), "g_val": np.arange(n, dtype=np.int64)}
+    exp = group_rows(G)
     dev = Q.upload_tables(ctx, {"G": G})
+
+    def read(r):
+        rows, cols = C.c_uint64(), C.c_int()
+        N.eng_check(eng.gdb_result_shape(r, C.byref(rows), C.byref(cols)))
+        out = np.zeros((cols.value, rows.value), np.int64)
+        N.eng_check(eng.gdb_result_words(r, out.ctypes.data))
+        return out
+
+    part = dict(variant="part", lds_slots=1024) if slots >= 65536 else dict(variant="global")
     try:
-        a = Q.run_groupby(ctx, dev, slots=2 * n, variant="part", lds_slots=1024)
-        first = {k: v.copy() for k, v in a.result.columns.items()}
-        b = Q.run_groupby(ctx, dev, slots=2 * n, variant="part", lds_slots=1024, val_cut=1000, executor=a.executor)
-        assert all(np.array_equal(a.result.columns[c], first[c]) for c in first)
-        assert np.array_equal(first["key"], np.arange(n)) and np.array_equal(np.sort(first["sum"]), np.arange(n))
+        a = Q.run_groupby(ctx, dev, slots=slots, **part)
+        held = []
+        for _ in range(2):
+            held.append(C.c_void_p())
+            N.eng_check(eng.gdb_executor_collect(a.executor.handle, a.plan.handle, C.byref(held[-1])))
+        b = Q.run_groupby(ctx, dev, slots=slots, val_cut=1000, executor=a.executor, **part)
         assert b.result.rows() == 1000
         a.executor.release()
+        a.executor.close()
+        for r in held:
+            for got, e in zip(read(r), exp.values()):
+                assert np.array_equal(got, e)
+            N.eng_check(eng.gdb_result_free(r))
     finally:
         dev["G"].free(ctx)

@@ -68,15 +68,44 @@ def test_partial_tables_take_the_room_the_rows_need(ctx):
             d["G"].free(ctx)
 
 
-def test_fold_of_a_chunked_run(ctx):
-    G = _table(500_000, 700, 5)
+# blocks of 4,096 rows against room for 512 partials (lds_slots 2048) or 256 (4096): several chunks' partials,
+# chunks of too few blocks to leave any, one chunk, and more partials than there is room for
+@pytest.mark.parametrize("n,chunk,lds_slots", [(500_000, 100_000, 2048), (500_000, 4096, 2048), (500_000, 500_000, 2048),
+                                               (1_400_000, 100_000, 4096)])
+def test_fold_of_a_chunked_run(ctx, n, chunk, lds_slots):
+    G = _table(n, 700, 5)
     h = E.HostTable("G", G)
     try:
-        for chunk in (100_000, 4096, 500_000):   # more partials than there is room for, one, and none left over
-            run = Q.run_groupby(ctx, {}, slots=2048, variant="lds", stream=Q.Stream(h, chunk))
-            _same(run.result.columns, G)
+        run = Q.run_groupby(ctx, {}, slots=2048, variant="lds", lds_slots=lds_slots, stream=Q.Stream(h, chunk))
+        _same(run.result.columns, G)
     finally:
         h.close()
+
+
+# 1, 3 partials for some 100 blocks a pipeline: the other blocks merge directly
+@pytest.mark.parametrize("partials", [1, 3])
+def test_more_blocks_than_partials(ctx, partials):
+    w = B.Workload3(ctx, B.workload3(n_pipes=8, scale=0.2, seed=79), lds_cap=4096, partials=partials)
+    try:
+        w.run_plain()
+        plain = w.results()
+        aggs = [s.index for s in w.specs if s.kind == "agg"]
+        blocks = []
+        for i in aggs:
+            blocks.append(w.execs[i].execute(w.batch_plans["agg"]).phases[0][2])
+            got = w.execs[i].collect(w.batch_plans["agg"]).columns
+            assert all(np.array_equal(got[k], plain[i][k]) for k in plain[i]), i
+        assert max(blocks) > 16
+        b = w.build_batch(512, 16_384)   # several work items a pipeline
+        try:
+            for _ in range(2):
+                b.run(graph=True)
+                for got, exp in zip(w.results(), plain):
+                    assert all(np.array_equal(got[k], exp[k]) for k in exp)
+        finally:
+            b.close()
+    finally:
+        w.close()
 
 
 @pytest.mark.parametrize("chunk", [2048, 20_000, 1 << 20])

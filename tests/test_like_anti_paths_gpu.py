@@ -1,7 +1,9 @@
 """LIKE '%w1%w2%' by the words' first four bytes: small alphabets, so heads
 match where words do not (the automata decide then), words of every length
-class, values ended by a NUL with bytes after it; and counts whose histogram
-crosses the register bins. Against the oracle, both signs."""
+class, words with a NUL in them (which match nothing, also where the bytes
+after a value's end hold them), values ended by a NUL with bytes after it; and
+counts whose histogram crosses the register bins. Against the oracle, both
+signs."""
 
 import numpy as np
 import pytest
@@ -11,7 +13,8 @@ from gpudbmetalcodegen_amd import queries as Q
 
 pytestmark = pytest.mark.gpu
 
-WORDS = [b"", b"a", b"ab", b"aba", b"abab", b"ababa", b"aaaab", b"abababab", b"baaaaaaab", b"ababababababababababab"]
+WORDS = [b"", b"a", b"ab", b"aba", b"abab", b"ababa", b"aaaab", b"abababab", b"baaaaaaab", b"ababababababababababab",
+         b"a\0", b"a\0a", b"aaaaa\0a"]
 
 
 @pytest.mark.parametrize("alphabet", [b"a", b"ab", b"abc"])
