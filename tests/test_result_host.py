@@ -1,6 +1,7 @@
-"""A result's large columns are copied by several threads; where threads cannot
-be created the copy still comes out whole. The collector's own source is built
-into a small program whose pthread_create fails from a given call on."""
+"""The host side of results, built from the collector's own source into small
+programs. A large column is copied by several threads, and still whole where
+threads cannot be created (pthread_create fails from a given call on). A group
+table that the device cannot order for want of memory is read and sorted here."""
 
 import subprocess
 from pathlib import Path
@@ -55,14 +56,58 @@ int main(int, char** argv) {
 """
 
 
-@pytest.fixture(scope="module")
-def program(tmp_path_factory):
-    d = tmp_path_factory.mktemp("copy")
-    (d / "main.cpp").write_text(PROGRAM)
+GROUPS = r"""
+#include "execution/hip_result_collector.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+int main(int, char** argv) {
+    using namespace gdb::codegen;
+    const uint64_t slots = std::strtoul(argv[1], nullptr, 10), groups = std::strtoul(argv[2], nullptr, 10);
+    std::vector<uint64_t> table(4 * slots, 0xFFFFFFFFull);
+    for (uint64_t g = 0; g < groups; ++g) {  // any slots, keys over the whole range
+        uint64_t* w = &table[4 * ((g * 7 + 3) % slots)];
+        w[0] = (g * 2654435761u & 0xFFFFFFFEull) | (g + 1) << 32;
+        w[1] = static_cast<uint64_t>(-static_cast<int64_t>(g));
+        w[2] = g;
+        w[3] = ~g;
+    }
+    HipResultSchema schema;
+    schema.kind = HipResultSchema::HASH_AGG;
+    schema.hash.tableName = "t";
+    schema.hash.slotsSymbol = "slots";
+    schema.hash.slotWords = 4;
+    const GenericResult r = HipResultCollector::collect(
+        schema,
+        [&](const std::string&, size_t off, void* dst, size_t bytes) {
+            std::memcpy(dst, reinterpret_cast<const char*>(table.data()) + off, bytes);
+        },
+        [&](const std::string&) { return slots; });
+    if (r.rows() != groups || r.columns.size() != 5) return 1;
+    for (size_t i = 0; i < groups; ++i) {
+        const int64_t g = r.columns[1].i64[i] - 1;
+        if (r.columns[0].i64[i] != static_cast<int64_t>(g * 2654435761u & 0xFFFFFFFEull)) return 2;
+        if (i && r.columns[0].i64[i] <= r.columns[0].i64[i - 1]) return 3;
+        if (r.columns[2].i64[i] != -g || r.columns[3].i64[i] != g || r.columns[4].i64[i] != ~g) return 4;
+    }
+    return 0;
+}
+"""
+
+
+def build(d: Path, source: str) -> Path:
+    (d / "main.cpp").write_text(source)
     subprocess.run(["g++", "-std=c++17", "-O1", f"-I{CSRC}", f"-I{CSRC.parent.parent / 'include'}", str(d / "main.cpp"),
                     str(CSRC / "execution" / "hip_result_collector.cpp"), str(CSRC / "core" / "hip_param_binding.cpp"),
                     "-o", str(d / "main"), "-pthread", "-ldl", "-rdynamic"], check=True)
     return d / "main"
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    return build(tmp_path_factory.mktemp("copy"), PROGRAM)
 
 
 # rows: one thread's share, the first size that is split, eight shares and one row more
@@ -73,3 +118,9 @@ def test_copy_without_threads(program, rows, threads):
     assert r.returncode == 0, r.stderr
     helpers = max(0, min(8, rows >> 18) - 1)
     assert int(r.stdout) == 2 * max(0, helpers - threads)
+
+
+def test_groups_sorted_on_the_host(tmp_path):
+    program = build(tmp_path, GROUPS)
+    for slots, groups in ((64, 0), (64, 1), (64, 64), (4096, 2000)):
+        assert subprocess.run([str(program), str(slots), str(groups)], timeout=60).returncode == 0, (slots, groups)
