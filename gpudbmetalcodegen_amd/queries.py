@@ -399,10 +399,19 @@ def run_q13(ctx: E.Context, dev: dict, w1: bytes, w2: bytes, negate: bool = Fals
     return QueryRun(res, t, plan, ex, st)
 
 
-# The anti-join marks referenced keys with byte flags from this many B rows on
-# (8M rows and 10% referencing: the atomic ORs of the bitmap cost 40 us more
-# than streaming the rows; the flags' extra packing launch costs 6 us, more
-# than they save in a smaller table), while the flags stay within the caches.
+# The anti-join marks referenced keys with byte flags from this many B rows on,
+# while the flags stay within the caches. Device us per run, atomic ORs against
+# flags, with 1%, 10% and all of the rows referencing (a share that is not known
+# before the scan):
+#   rows   keys   1%           10%          all
+#   1M     0.1M   23.7 / 31.0  31.2 / 30.5  103 / 33
+#   4M     0.4M   28.3 / 33.2  45.8 / 34.6  210 / 50
+#   8M     0.8M   39.2 / 40.1  69.4 / 44.3  408 / 74
+#   8M     8M     71.8 / 80.5  96.1 / 90.6  366 / 202
+#   30M    3M     87.6 / 83.5  167 / 117    1196 / 398
+#   30M    30M    218 / 227    295 / 256    1292 / 830
+# A smaller table loses its 6.5 us of packing where few rows reference and gains
+# where many do; from 8M rows on only dense keys that few rows reference lose.
 Q22_FLAG_ROWS = 8_000_000
 Q22_FLAG_KEYS = 64 << 20
 
