@@ -102,9 +102,10 @@ gdb_status gdb_executor_register_symbol(gdb_executor ex, const char* name, uint6
 gdb_status gdb_executor_get_symbol(gdb_executor ex, const char* name, uint64_t* value, int* found);
 gdb_status gdb_executor_register_scalar(gdb_executor ex, const char* name, int64_t value);
 gdb_status gdb_executor_set_skip_init(gdb_executor ex, int skip);
-// on = 1 (default): gdb_exec_timing holds every phase's device time (an event
-// pair around each phase); on = 0: only the whole run's (one event at each
-// end), for runs that need no breakdown. No counterpart in the reference,
+// on = 1 (default): gdb_exec_timing holds every phase's device time, from the
+// end of the phase before it, so with the gap between the two launches, or from
+// its own start where fills or a hook lie between; on = 0: only the whole run's
+// (one event at each end), for runs that need no breakdown. No counterpart in the reference,
 // whose timings come from command-buffer timestamps
 // (codegen/execution/metal_generic_executor.cpp:338-390).
 gdb_status gdb_executor_set_phase_timing(gdb_executor ex, int on);
@@ -169,6 +170,10 @@ gdb_status gdb_executor_enqueue(gdb_executor ex, gdb_plan p);
 gdb_status gdb_executor_check_status(gdb_executor ex, gdb_plan p);
 gdb_status gdb_executor_read_buffer(gdb_executor ex, const char* name, size_t offset, void* host, size_t bytes);
 gdb_status gdb_executor_buffer_ptr(gdb_executor ex, const char* name, void** dptr, size_t* bytes);
+/* Device memory of the runner: its buffers, and up to 2 GiB of workspace kept
+ * from large group-by results. Besides, a runner keeps up to 256 MiB of
+ * page-locked host memory that its last large result was read into.
+ * gdb_executor_release gives back what no open result holds. */
 gdb_status gdb_executor_owned_bytes(gdb_executor ex, size_t* bytes);
 gdb_status gdb_executor_release(gdb_executor ex);
 
