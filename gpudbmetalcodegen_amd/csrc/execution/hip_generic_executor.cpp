@@ -65,11 +65,13 @@ void HipGenericExecutor::syncStream() {
 }
 
 void HipGenericExecutor::registerTable(const std::string& table, uint64_t rows) {
-    tables_[table].rows = rows;
+    TableInfo& t = tables_[table];
+    t.rows = rows;
     sizes_.registerSymbol(tableSizeName(table), rows);
-    uint64_t most = 0;
-    tryGetSymbol(tableMaxSizeName(table), most);
-    sizes_.registerSymbol(tableMaxSizeName(table), std::max(most, rows));
+    if (t.registered && rows <= t.mostRows) return;
+    t.registered = true;
+    t.mostRows = rows;
+    sizes_.registerSymbol(tableMaxSizeName(table), rows);
 }
 
 void HipGenericExecutor::registerTableColumn(const std::string& table, const std::string& column, const void* devptr) {
@@ -504,8 +506,8 @@ HipExecutionResult HipGenericExecutor::execute(RuntimeCompiler& rc, const Runtim
             const size_t e = static_cast<size_t>(2 * (pi - firstPhase));
             bool marked = apart;
             bool foldFollows = p.partialsSymbol.empty() || p.foldsPartials;
-            for (int f = pi + 1; f < last; ++f)
-                foldFollows |= phases[static_cast<size_t>(f)].partialsSymbol == p.partialsSymbol;
+            for (int f = pi + 1; f < last && !foldFollows; ++f)
+                foldFollows = phases[static_cast<size_t>(f)].partialsSymbol == p.partialsSymbol;
             launchPhase(rc, cq, p, initDone, spec, foldFollows, &grid, phaseTiming_ ? events_[e + 1] : nullptr, &marked);
             ownStart_[static_cast<size_t>(pi - firstPhase)] = marked;
             apart = false;

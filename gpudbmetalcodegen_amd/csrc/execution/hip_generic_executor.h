@@ -170,6 +170,8 @@ private:
     };
     struct TableInfo {
         uint64_t rows = 0;
+        uint64_t mostRows = 0;
+        bool registered = false;
         std::unordered_map<std::string, const void*> columns;
     };
     struct BufferTable {
