@@ -655,20 +655,33 @@ gdb_status gdb_result_column_format(gdb_result r, int idx, int* scale, int* is_d
     return GDB_OK;
 }
 
+// Column idx of a result when it is of `type`; null, with the error set, when
+// there is no such column.
+static const ResultColumn* resultColumn(gdb_result r, int idx, ResultColumn::Type type, const char* call, const char* kind) {
+    if (idx < 0 || idx >= static_cast<int>(r->r.columns.size())) {
+        setErr(GDB_ERR_INVALID, std::string(call) + ": index out of range");
+        return nullptr;
+    }
+    const auto& c = r->r.columns[static_cast<size_t>(idx)];
+    if (c.type == type) return &c;
+    setErr(GDB_ERR_INVALID, std::string(call) + ": column is not " + kind);
+    return nullptr;
+}
+
 gdb_status gdb_result_i64(gdb_result r, int idx, int64_t* out) {
-    const auto& c = r->r.columns.at(static_cast<size_t>(idx));
-    if (c.type != ResultColumn::I64) return setErr(GDB_ERR_INVALID, "gdb_result_i64: column is not int64");
     return guard([&]() -> gdb_status {
-        c.copyI64(out);
+        const auto* c = resultColumn(r, idx, ResultColumn::I64, "gdb_result_i64", "int64");
+        if (!c) return GDB_ERR_INVALID;
+        c->copyI64(out);
         return GDB_OK;
     });
 }
 
 gdb_status gdb_result_i128(gdb_result r, int idx, int64_t* out) {
-    const auto& c = r->r.columns.at(static_cast<size_t>(idx));
-    if (c.type != ResultColumn::I128) return setErr(GDB_ERR_INVALID, "gdb_result_i128: column is not int128");
-    for (size_t i = 0; i < c.i128.size(); ++i) {
-        const unsigned __int128 u = static_cast<unsigned __int128>(c.i128[i]);
+    const auto* c = resultColumn(r, idx, ResultColumn::I128, "gdb_result_i128", "int128");
+    if (!c) return GDB_ERR_INVALID;
+    for (size_t i = 0; i < c->i128.size(); ++i) {
+        const unsigned __int128 u = static_cast<unsigned __int128>(c->i128[i]);
         out[2 * i] = static_cast<int64_t>(static_cast<uint64_t>(u));
         out[2 * i + 1] = static_cast<int64_t>(static_cast<uint64_t>(u >> 64));
     }
@@ -676,11 +689,11 @@ gdb_status gdb_result_i128(gdb_result r, int idx, int64_t* out) {
 }
 
 gdb_status gdb_result_str(gdb_result r, int idx, char* out, size_t width) {
-    const auto& c = r->r.columns.at(static_cast<size_t>(idx));
-    if (c.type != ResultColumn::STR) return setErr(GDB_ERR_INVALID, "gdb_result_str: column is not a string");
-    for (size_t i = 0; i < c.str.size(); ++i) {
+    const auto* c = resultColumn(r, idx, ResultColumn::STR, "gdb_result_str", "a string");
+    if (!c) return GDB_ERR_INVALID;
+    for (size_t i = 0; i < c->str.size(); ++i) {
         std::memset(out + i * width, 0, width);
-        std::memcpy(out + i * width, c.str[i].data(), std::min(width, c.str[i].size()));
+        std::memcpy(out + i * width, c->str[i].data(), std::min(width, c->str[i].size()));
     }
     return GDB_OK;
 }

@@ -3,9 +3,12 @@ Python from the columns and formats, over results with fixed-point, 128-bit,
 negative, date and string columns, extreme values, no rows, and labels that
 hold the separators of the one-call description."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from gpudbmetalcodegen_amd import _native as N
 from gpudbmetalcodegen_amd import queries as Q
 from gpudbmetalcodegen_amd import tpch as T
 from gpudbmetalcodegen_amd import tpch_gen as G
@@ -81,3 +84,27 @@ def test_extreme_values_text(ctx):
         assert res.canonical == _text(res)
     finally:
         dev["G"].free(ctx)
+
+
+def test_column_calls_refuse_other_columns(ctx):
+    """Indexes outside the result and columns of another type are errors."""
+    dev = Q.upload_tables(ctx, W.workload0(5000))
+    eng, r = N.load()[1], C.c_void_p()
+    try:
+        run = Q.run_q1(ctx, dev, W.q1_cutoff())
+        N.eng_check(eng.gdb_executor_collect(run.executor.handle, run.plan.handle, C.byref(r)))
+        rows, cols = run.result.rows(), len(run.result.columns)
+        out = np.zeros(2 * rows, np.int64)
+        types = []
+        for i in range(cols):
+            got = (eng.gdb_result_i64(r, i, out.ctypes.data), eng.gdb_result_i128(r, i, out.ctypes.data),
+                   eng.gdb_result_str(r, i, C.create_string_buffer(64 * rows), 64))
+            assert sorted(got) == [N.GDB_OK, N.GDB_ERR_INVALID, N.GDB_ERR_INVALID]
+            types.append(got.index(N.GDB_OK))
+        assert set(types) == {0, 1, 2}
+        for i in (-1, cols):
+            for st in (eng.gdb_result_i64(r, i, None), eng.gdb_result_i128(r, i, None), eng.gdb_result_str(r, i, None, 64)):
+                assert st == N.GDB_ERR_INVALID and b"index out of range" in eng.gdb_engine_last_error()
+        N.eng_check(eng.gdb_result_free(r))
+    finally:
+        dev["F"].free(ctx)
